@@ -227,7 +227,7 @@ def bench_cfg4(D, S, prng, steps=5):
                 D.lib.smith_matmul_q4(D.ops_ctx(), a.buffer, W.bufs[i % len(W.bufs)], out.buffer, M, Nn, Kk,
                                       (Kk + 31) // 32)
             kms, kn = D.profile_read("smith_gemm_q4s")
-            kms2, kn2 = D.profile_read("smith_gemm2_q4s")  # the DMA-staged kernels
+            kms2, kn2 = D.profile_read("smith_gemm3_q4s")  # the DMA-staged kernels
             kms, kn = kms + kms2, kn + kn2
             D.profile_read("")  # drop the other records (activation prep, reduce)
             D.profile_kernels(False)
@@ -238,7 +238,7 @@ def bench_cfg4(D, S, prng, steps=5):
                 "ms_step": round(msx, 3), "kernels_per_step": ktx["launches_per_step"],
                 "gemm_kernel_us": round(kus, 1), "gemm_kernel_TFLOPs": round(fl / kus / 1e6, 1),
                 "gemm_kernel_mfma_util": round(fl / kus / 1e6 / MFMA_F16_PEAK_TFLOPS, 4),
-                "path": "f16 activation prep + MFMA GEMM (Q4S dequantized to f16 in LDS, f32 accumulation)"}
+                "path": "f16 activation prep + MFMA GEMM (Q4S dequantized to f16 in registers, f32 accumulation)"}
             log("cfg4 M=%d N=%d K=%d:" % (M, Nn, Kk), pre["M%d_N%d_K%d" % (M, Nn, Kk)])
     return pre
 

@@ -8,6 +8,8 @@
 //                       q50t, q4kt, q6kt}
 //   smith_gemm_prep_a_perm + smith_gemm2_<fmt>_m<BM>_n<BN>  the DMA-staged
 //                       GEMM for the tile-plane formats (further below)
+//   smith_gemm3_<fmt>_m<TM>  the DMA-staged GEMM for the record formats (q4s,
+//                       q8, q40) with K % 64 == 0
 //
 // Workgroup tile BM x BN (128x64 .. 256x256), K in stages of BK=64 (two
 // 32-row quantization groups), double-buffered in LDS: while the MFMAs
@@ -710,6 +712,356 @@ DEF_GEMM2_FMT(q41t, GT_Q41)
 DEF_GEMM2_FMT(q50t, GT_Q50)
 DEF_GEMM2_FMT(q4kt, GT_Q4K)
 DEF_GEMM2_FMT(q6kt, GT_Q6K)
+
+// ---------------------------------------------------------------------------
+// gemm3: the GEMM on (g, n) records (Q4S, Q8, Q4_0 planes), K % 64 == 0.
+// Workgroup tile 16*TM rows x 256 columns, eight waves side by side along N,
+// each over all the rows and 32 columns.  Stages of K = 64 in a ring of three
+// LDS buffers filled by 16-byte direct-to-LDS loads: the A rows (16-byte
+// chunks XOR-swizzled by row through each lane's source address) and the two
+// groups' raw records, which are contiguous over the tile's columns.  A wave
+// converts the records of its own columns to f16 in registers beside its
+// MFMAs, so a weight is converted once per workgroup and never written back
+// to LDS.  The MFMA takes the weights as its A operand: a lane then holds four
+// consecutive output columns of one row, so a tile is stored with 16-byte
+// stores and a SwiGLU pair sits in one lane.
+//
+// What bounds it: the card's power.  On zero activations the same launches
+// take 13-25 % less time, and MFMAs alone on random f16 operands reach 1630
+// TFLOP/s (2216 on constant ones), so what counts is work per MFMA: the
+// conversion (11-19 % of the time when left out) and the LDS traffic.  Two
+// waves along M converted each weight twice (Q8, M = 301: 61.6 us instead of
+// 50.1); four waves of 256 x 64 spill.
+// Measured (whole call: activation prep, GEMM, K-split reduce; the register-
+// staged kernel before it): Q4S M = 512, 14336 x 4096 80 -> 66 us; M = 2048,
+// 4096 x 14336 259 -> 242 us; Q8 M = 301, 14336 x 4096 84 -> 57 us.
+// ---------------------------------------------------------------------------
+// 16 bytes per lane from base + off (a lane's own) to LDS byte address lds +
+// 16 * lane (wave-uniform).  In asm so that the compiler does not see an LDS
+// write: it would wait for every load in flight before the next LDS read.
+// There is no destination register, and the kernel counts the loads itself
+// (s_waitcnt vmcnt before the barrier that publishes a stage).  One wait
+// state between the write of M0 and its use.
+__device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2"
+      :
+      : "s"(lds), "v"(off), "s"(base)
+      : "memory", "m0");
+}
+
+// a wave-uniform 64-bit value in scalar registers
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return (uint64_t)hi << 32 | lo;
+}
+
+template <int FMT, int TM>
+struct G3 {
+  static constexpr int NW = 8, TN = 2, BM = 16 * TM, BN = 16 * TN * NW;
+  static constexpr int R = FMT == WF_Q4S ? 24 : (FMT == WF_Q8 ? 34 : 16);  // bytes of a record in B
+  static constexpr bool HAS_D = FMT == WF_Q40;
+  static constexpr int A_CH = BM / 8;  // 1 KB chunks: 8 rows of 128 B
+  // records of one group, plus up to 3 bytes below a 4-byte aligned start
+  static constexpr int RCH = (BN * R + (R % 4 ? 3 : 0) + 1023) / 1024, RUN = RCH * 1024;
+  static constexpr int DCH = HAS_D ? 1 : 0;  // BN f16 scales of one group
+  static constexpr int B_CH = 2 * (RCH + DCH);
+  static constexpr int A_PW = (A_CH + NW - 1) / NW, B_PW = (B_CH + NW - 1) / NW, CNT = A_PW + B_PW;  // loads per wave and stage
+  static constexpr int STAGE = (A_CH + B_CH) * 1024;
+  static_assert(BN * 2 + 3 <= 1024, "one chunk of scales");
+};
+
+// Schedule hint for the block of code before it: after each of N MFMAs one
+// LDS read and V vector instructions, so that a wave's conversions and reads
+// issue in the shadow of its own MFMAs (measured against the compiler's own
+// order and against groups of 2 and 4 MFMAs: 128 x 256 tiles of Q4S 76.7 ->
+// 74.9 us, 160 x 256 of Q8 56.4 -> 50.1 us)
+template <int N, int V>
+__device__ __forceinline__ void g3_interleave() {
+#pragma unroll
+  for (int q = 0; q < N; q++) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+  }
+}
+
+template <uint32_t V>
+struct KeepStages {
+  static constexpr uint32_t value = V;
+};
+
+// what a lane reads from LDS for eight weights of one column
+template <int FMT>
+struct G3Raw {
+  uint32_t x[FMT == WF_Q8 ? 3 : 1];
+  float s, z;
+};
+
+template <int FMT, int TM>
+__device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, const uint8_t* __restrict__ B,
+                                          const uint16_t* __restrict__ D, float* __restrict__ C, uint32_t M,
+                                          uint32_t N, uint32_t K, const float* __restrict__ R, uint32_t epi,
+                                          float* __restrict__ ws, uint32_t sps) {
+  using P = G3<FMT, TM>;
+  constexpr int BM = P::BM, BN = P::BN, TN = P::TN;
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[3 * P::STAGE];
+
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t MB = (M + BM - 1) / BM, NBk = (N + BN - 1) / BN, T = MB * NBk;
+  // XCD x (= id % 8) takes a contiguous run of tiles, M fastest, so the
+  // tiles that share weights run on one L2
+  const uint32_t xq = T / 8, xr = T % 8, xcd = blockIdx.x % 8, xi = blockIdx.x / 8;
+  const uint32_t t = xcd * xq + (xcd < xr ? xcd : xr) + xi;
+  const uint32_t nb = t / MB, mb = t % MB;
+  const uint32_t m0 = mb * BM, n0 = nb * BN;
+  const uint32_t Sall = K / 64;
+  const uint32_t s0 = blockIdx.y * sps < Sall ? blockIdx.y * sps : Sall;
+  const uint32_t s1 = s0 + sps < Sall ? s0 + sps : Sall;
+  const uint32_t S = s1 - s0;
+
+  // sources of this wave's loads: a uniform base per load, advanced by a
+  // uniform stride per stage, plus a per-lane offset formed once.  A wave
+  // past the last chunk loads the last one again (same bytes, same place).
+  uint32_t va[P::A_PW], vb[P::B_PW];
+  uint32_t lb[P::B_PW];
+  const uint8_t* pb[P::B_PW];
+  size_t strb[P::B_PW];
+  const uint8_t* pa = (const uint8_t*)(A16 + (size_t)m0 * K + (size_t)s0 * 64);
+#pragma unroll
+  for (int i = 0; i < P::A_PW; i++) {
+    const uint32_t j = wave + P::NW * i < (uint32_t)P::A_CH ? wave + P::NW * i : (uint32_t)P::A_CH - 1;
+    const uint32_t row = 8 * j + (lane >> 3), c = (lane & 7) ^ (row & 7);
+    const uint32_t m = m0 + row < M ? row : M - 1 - m0;
+    va[i] = m * K * 2 + c * 16;
+  }
+  const uint32_t valid = N - n0 < (uint32_t)BN ? N - n0 : BN;
+  // byte offset of group gi's first record above its 4-byte aligned start
+  uint32_t shq[2], shd[2];
+#pragma unroll
+  for (int gi = 0; gi < 2; gi++) {
+    shq[gi] = P::R % 4 ? (uint32_t)((size_t)B + ((size_t)gi * N + n0) * P::R) & 3u : 0u;
+    shd[gi] = P::HAS_D ? (uint32_t)((size_t)D + ((size_t)gi * N + n0) * 2) & 3u : 0u;
+  }
+#pragma unroll
+  for (int i = 0; i < P::B_PW; i++) {
+    const uint32_t j = wave + P::NW * i < (uint32_t)P::B_CH ? wave + P::NW * i : (uint32_t)P::B_CH - 1;
+    const bool isd = P::HAS_D && j >= 2 * P::RCH;
+    const uint32_t gi = isd ? j - 2 * P::RCH : j / P::RCH;
+    const uint32_t rec = isd ? 2u : (uint32_t)P::R, sh = isd ? (gi ? shd[1] : shd[0]) : (gi ? shq[1] : shq[0]);
+    const uint32_t off = (isd ? 0u : (j % P::RCH) * 1024) + lane * 16;
+    const uint32_t last = (valid * rec + sh - 1) & ~15u;  // the 16 bytes that hold the run's last byte
+    vb[i] = off < last ? off : last;
+    pb[i] = (const uint8_t*)uniform64((size_t)(isd ? (const uint8_t*)D : B) + ((size_t)(2 * s0 + gi) * N + n0) * rec - sh);
+    strb[i] = uniform64((size_t)2 * N * rec);
+    lb[i] = j * 1024;
+  }
+  const uint32_t lds0 = (uint32_t)(size_t)(lds_ptr_t)ring;
+  auto issue = [&](uint32_t s, uint32_t buf) {  // stage s0 + s into the buffer at byte buf of the ring
+#pragma unroll
+    for (int i = 0; i < P::A_PW; i++) {
+      const uint32_t j = wave + P::NW * i < (uint32_t)P::A_CH ? wave + P::NW * i : (uint32_t)P::A_CH - 1;
+      dma16(pa + (size_t)s * 128, va[i], lds0 + buf + j * 1024);
+    }
+#pragma unroll
+    for (int i = 0; i < P::B_PW; i++) dma16(pb[i] + s * strb[i], vb[i], lds0 + buf + P::A_CH * 1024 + lb[i]);
+  };
+
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const uint32_t r16 = lane & 15, kq = lane >> 4;
+
+  // exponent bits of the nibble conversion, kept in registers: one v_and_or
+  // a pair instead of two instructions with a literal each
+  uint32_t e1024 = 0x64006400u, e64 = 0x54005400u;
+  asm volatile("" : "+v"(e1024), "+v"(e64));
+  const uint32_t bcol = wave * 16 * TN + r16;
+  // the fields of column bcol + 16 j, K slice 8 kq .. +7, of group kk of a stage
+  auto raw = [&](const uint8_t* bs, int j, int kk) {
+    G3Raw<FMT> w;
+    const uint32_t col = bcol + 16 * j;
+    if constexpr (FMT == WF_Q8) {
+      const uint32_t o = kk * P::RUN + shq[kk] + col * 34;
+      const uint32_t* p = (const uint32_t*)(bs + ((o + 2 + 8 * kq) & ~3u));
+      w.x[0] = p[0];
+      w.x[1] = p[1];
+      w.x[2] = p[2];
+      w.s = (float)*(const _Float16*)(bs + o);
+    } else {
+      const uint8_t* p = bs + kk * P::RUN + col * P::R;
+      w.x[0] = *(const uint32_t*)(p + 4 * kq);
+      if constexpr (FMT == WF_Q4S) {
+        const float2 sz = *(const float2*)(p + 16);
+        w.s = sz.x;
+        w.z = sz.y;
+      } else {
+        w.s = (float)*(const _Float16*)(bs + 2 * P::RUN + kk * 1024 + shd[kk] + col * 2);
+      }
+    }
+    return w;
+  };
+  auto weight = [&](const G3Raw<FMT>& w, int j, int kk) -> half8 {
+    if constexpr (FMT == WF_Q8) {
+      const uint32_t a = (shq[kk] + (bcol + 16 * j) * 34 + 2) & 3u;
+      const uint32_t x0 = __builtin_amdgcn_alignbyte(w.x[1], w.x[0], a) ^ 0x80808080u;
+      const uint32_t x1 = __builtin_amdgcn_alignbyte(w.x[2], w.x[1], a) ^ 0x80808080u;
+      // bytes b + 128 as f16 1024 + (b + 128); 1152 comes off exactly, one rounding by the scale
+      const h2 off = {(_Float16)1152.0f, (_Float16)1152.0f}, s2 = {(_Float16)w.s, (_Float16)w.s};
+      u32x4 u;
+      u.x = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(h2, __builtin_amdgcn_perm(e1024, x0, 0x05010500u)) - off) * s2);
+      u.y = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(h2, __builtin_amdgcn_perm(e1024, x0, 0x05030502u)) - off) * s2);
+      u.z = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(h2, __builtin_amdgcn_perm(e1024, x1, 0x05010500u)) - off) * s2);
+      u.w = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(h2, __builtin_amdgcn_perm(e1024, x1, 0x05030502u)) - off) * s2);
+      return __builtin_bit_cast(half8, u);
+    } else {
+      // nibbles in the slot order {0,4,1,5,2,6,3,7} (A is prepared alike), as q4_pairs
+      const uint32_t x = w.x[0], y = x >> 8;
+      const _Float16 sh = (_Float16)w.s, ch = FMT == WF_Q4S ? (_Float16)(-w.s * w.z) : sh * (_Float16)(-8.0f);  // -8 d exact
+      const h2 sv = {sh, sh}, cv = {ch, ch};
+      const h2 blo = (h2){(_Float16)1024.0f, (_Float16)1024.0f}, bhi = (h2){(_Float16)64.0f, (_Float16)64.0f};
+      const h2 v0 = __builtin_elementwise_fma(__builtin_bit_cast(h2, (x & 0x000F000Fu) | e1024) - blo, sv, cv);
+      const h2 v1 = __builtin_elementwise_fma(__builtin_bit_cast(h2, (x & 0x00F000F0u) | e64) - bhi, sv, cv);
+      const h2 v2 = __builtin_elementwise_fma(__builtin_bit_cast(h2, (y & 0x000F000Fu) | e1024) - blo, sv, cv);
+      const h2 v3 = __builtin_elementwise_fma(__builtin_bit_cast(h2, (y & 0x00F000F0u) | e64) - bhi, sv, cv);
+      const u32x4 u = {__builtin_bit_cast(uint32_t, v0), __builtin_bit_cast(uint32_t, v1),
+                       __builtin_bit_cast(uint32_t, v2), __builtin_bit_cast(uint32_t, v3)};
+      return __builtin_bit_cast(half8, u);
+    }
+  };
+
+  // Ring of three buffers.  Once every wave holds the last A rows of stage s
+  // in registers (the barrier between the two halves of its second group's
+  // MFMAs), stage s + 3 goes into its buffer and the first weights of stage
+  // s + 1 are converted beside the MFMAs that are left: a stage has two
+  // stages' time to arrive, and no MFMA waits for a conversion.  Past the end
+  // the last stage is loaded again, which nothing reads, so the wait is one
+  // constant.
+  if (S > 0) {
+    auto landed = [&](auto keep) { __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(keep)::value * P::CNT)); };
+    issue(0, 0);
+    issue(S > 1 ? 1 : 0, P::STAGE);
+    issue(S > 2 ? 2 : S - 1, 2 * P::STAGE);
+    const uint32_t aoff = r16 * 128;
+        constexpr int H = TM / 2;  // row tiles of the second group's MFMAs before the barrier
+    uint32_t cur = 0;
+    half8 b0[TN], b1[TN];
+    G3Raw<FMT> w[TN];
+    landed(KeepStages<2>{});
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int j = 0; j < TN; j++) b0[j] = weight(raw(ring + P::A_CH * 1024, j, 0), j, 0);
+    for (uint32_t s = 0; s < S; s++) {
+      const uint8_t* as = ring + cur;
+      half8 af[TM];
+#pragma unroll
+      for (int i = 0; i < TM; i++) af[i] = *(const half8*)(as + aoff + i * 2048 + 16 * (kq ^ (r16 & 7)));
+#pragma unroll
+      for (int j = 0; j < TN; j++) w[j] = raw(as + P::A_CH * 1024, j, 1);
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0[j], af[i], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < TN; j++) b1[j] = weight(w[j], j, 1);
+      half8 ag[TM];
+#pragma unroll
+      for (int i = 0; i < TM; i++) ag[i] = *(const half8*)(as + aoff + i * 2048 + 16 * ((4 + kq) ^ (r16 & 7)));
+#pragma unroll
+      for (int i = 0; i < H; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b1[j], ag[i], acc[i][j], 0, 0, 0);
+      g3_interleave<(TM + H) * TN, 1>();
+      // every LDS read of stage s is done, stage s + 1 has landed
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      landed(KeepStages<1>{});
+      __builtin_amdgcn_s_barrier();
+      issue(s + 3 < S ? s + 3 : S - 1, cur);
+      cur = cur == 2 * P::STAGE ? 0 : cur + P::STAGE;
+#pragma unroll
+      for (int j = 0; j < TN; j++) w[j] = raw(ring + cur + P::A_CH * 1024, j, 0);
+#pragma unroll
+      for (int i = H; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b1[j], ag[i], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < TN; j++) b0[j] = weight(w[j], j, 0);
+      g3_interleave<(TM - H) * TN, 2>();
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // nothing may land in LDS after the workgroup has ended
+  }
+
+  const bool split = gridDim.y > 1;
+  const uint32_t ldc = !split && epi == 2 ? N / 2 : N;
+  float* out = split ? ws + (size_t)blockIdx.y * M * N : C;
+  const bool vec = N % 4 == 0 && ((size_t)out & 15) == 0 && (split || epi != 1 || ((size_t)R & 15) == 0);
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+    const uint32_t m = m0 + i * 16 + r16;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const uint32_t n = n0 + wave * 16 * TN + j * 16 + 4 * kq;
+      if (n >= N) continue;
+      f32x4 v = acc[i][j];
+      if (!split && epi == 2) {  // (gate, up) at columns 2c, 2c+1
+        float* o = out + (size_t)m * ldc + n / 2;
+        const float y0 = silu_mul_g(v[0], v[1]), y1 = silu_mul_g(v[2], v[3]);
+        if (vec) {
+          *(float2*)o = make_float2(y0, y1);
+        } else {
+          if (n + 1 < N) o[0] = y0;
+          if (n + 3 < N) o[1] = y1;
+        }
+        continue;
+      }
+      float* o = out + (size_t)m * ldc + n;
+      const float* r = R + (size_t)m * N + n;
+      if (vec) {
+        if (!split && epi == 1) {
+          const float4 rv = *(const float4*)r;
+          v = (f32x4){v[0] + rv.x, v[1] + rv.y, v[2] + rv.z, v[3] + rv.w};
+        }
+        *(float4*)o = make_float4(v[0], v[1], v[2], v[3]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (n + e < N) o[e] = !split && epi == 1 ? v[e] + r[e] : v[e];
+      }
+    }
+  }
+}
+
+#define DEF_GEMM3(TAG, FMT, TM)                                                                              \
+  extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))                        \
+  void smith_gemm3_##TAG##_m##TM(                                                                             \
+      const _Float16* __restrict__ A16, const uint8_t* __restrict__ B, const uint16_t* __restrict__ D,       \
+      float* __restrict__ C, uint32_t M, uint32_t N, uint32_t K, const float* __restrict__ R, uint32_t epi,   \
+      float* __restrict__ ws, uint32_t sps) {                                                                \
+    gemm3_body<FMT, TM>(A16, B, D, C, M, N, K, R, epi, ws, sps);                                              \
+  }
+// 16 * TM rows a workgroup (the bridge picks TM so that the rows split evenly)
+#define DEF_GEMM3_FMT(TAG, FMT) \
+  DEF_GEMM3(TAG, FMT, 4)        \
+  DEF_GEMM3(TAG, FMT, 6)        \
+  DEF_GEMM3(TAG, FMT, 8)        \
+  DEF_GEMM3(TAG, FMT, 10)       \
+  DEF_GEMM3(TAG, FMT, 12)       \
+  DEF_GEMM3(TAG, FMT, 14)       \
+  DEF_GEMM3(TAG, FMT, 16)
+DEF_GEMM3_FMT(q4s, WF_Q4S)
+DEF_GEMM3_FMT(q8, WF_Q8)
+DEF_GEMM3_FMT(q40, WF_Q40)
 
 template <bool PERM>
 __device__ __forceinline__ void prep_a_row(const float* __restrict__ A, const float* __restrict__ gamma, float eps,

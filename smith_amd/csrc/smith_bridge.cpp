@@ -533,6 +533,43 @@ int qgemv1_chunk(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, 
 // weights dequantized to f16 in LDS, MFMA GEMM with f32 accumulation.
 const uint32_t GEMM_MIN_M = 64;
 
+// sizes of the static scratch of smith_matmul_q4_noalloc (layout at its definition)
+constexpr size_t NOALLOC_BYTES = 32u << 20;
+constexpr size_t NOALLOC_CNT_BYTES = 64u << 10;
+constexpr size_t NOALLOC_PREP_BYTES = 4u << 20;
+
+// Row tiles per workgroup (TM) and K splits of smith_gemm3_*: the pair with
+// the least estimated time.  256 workgroups run at once (one a CU); a stage
+// of K = 64 takes about 0.35 + 0.076 TM us (Q8, whose conversion is longer,
+// 0.45), filling the ring and storing the tile 3 + 0.35 TM us, and splits add
+// the reduce: partials read and result written at 7.2 TB/s, and 5 us.
+// (Measured on either side: Q4S M = 512, 14336 x 4096 TM = 8 without splits
+// 71 us, 16 with two 81; Q8 M = 301 10 with two 61, 8 without 69; Q4S M =
+// 2048, 4096 x 14336 both 252.)
+uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, uint32_t* ks_out) {
+  const double conv = fmt == FQ8 ? 0.45 : 0.35;
+  static const uint32_t tms[] = {4, 6, 8, 10, 12, 14, 16};
+  double best = 1e30;
+  uint32_t btm = 16;
+  *ks_out = 1;
+  for (uint32_t tm : tms) {
+    const uint64_t tiles = (uint64_t)((M + 16 * tm - 1) / (16 * tm)) * ((N + 255) / 256);
+    for (uint32_t ks = 1; ks <= 16 && (ks == 1 || S / ks >= 4); ks++) {
+      const uint32_t sps = (S + ks - 1) / ks;
+      if ((S + sps - 1) / sps != ks) continue;  // the same stages per split as a smaller count
+      // the static scratch takes every plan of the shapes whose activations
+      // it holds, so that both matmulQ4 entry points run the same one
+      if (ks > 1 && fmt == FQ4S && (size_t)M * S * 128 <= NOALLOC_PREP_BYTES &&
+          (size_t)ks * M * N * sizeof(float) > NOALLOC_BYTES - NOALLOC_CNT_BYTES - NOALLOC_PREP_BYTES)
+        break;
+      double t = (double)((tiles * ks + 255) / 256) * (sps * (conv + 0.076 * tm) + 3.0 + 0.35 * tm);
+      if (ks > 1) t += 5.0 + (ks + 1.0) * M * N * 4.0 / 7.2e6;
+      if (t < best) best = t, btm = tm, *ks_out = ks;
+    }
+  }
+  return btm;
+}
+
 int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* out, uint32_t M, uint32_t N,
          uint32_t K, const Epi& ep) {
   // A operand already written by the previous GEMM's fused reduce (same
@@ -554,6 +591,8 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
     return !(e && e[0] == '0');
   }();
   const bool g2 = gemm2_on && (fmt == FQ40T || fmt >= FQ41T) && K % 64 == 0;
+  const bool g3 = (fmt == FQ4S || fmt == FQ8 || fmt == FQ40) && K % 64 == 0 &&
+                  ((uintptr_t)B & (fmt == FQ8 ? 1 : 3)) == 0 && ((uintptr_t)D & 1) == 0;
   {
     const float* pa = a;
     const float* pg = ep.gamma;
@@ -579,12 +618,10 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
   if (g2 && bm == 256 && bn == 256) bn = 128;  // 256x256 spills registers on the high-bit formats
   // M >= 256 on the register-staged kernel: 256x256 tiles (one 1024-thread
   // workgroup per CU) and enough K splits to fill one wave of workgroups,
-  // each split at least 8 stages -- measured best at config 4 (M = 512:
-  // 123 -> 114 us at K = 4096, 191 -> 110 us at K = 14336; M = 2048,
-  // K = 14336: 411 -> 359 us; M = 2048, K = 4096 unchanged)
+  // each split at least 8 stages
   const bool big = !g2 && M >= 256;
   if (big) bm = bn = 256;
-  const uint32_t tiles = ntiles(bm, bn);
+  uint32_t tiles = ntiles(bm, bn);
   const uint32_t S = (K + 63) / 64;
   uint32_t ks = 1;
   if (big) {
@@ -595,12 +632,22 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
   } else if (bm == 128 && bn == 64 && tiles < 512) {
     ks = std::min<uint32_t>((512 + tiles - 1) / tiles, std::max<uint32_t>(1, S / 8));
   }
-  const uint32_t sps = (S + ks - 1) / ks;
+  uint32_t sps = (S + ks - 1) / ks;
   ks = (S + sps - 1) / sps;
   if (ks > 1 && ensure(c, (void**)&c->ws, &c->ws_bytes, (size_t)ks * M * N * sizeof(float))) return -1;
-  const uint32_t threads = 64 * (bm / 64) * (bn / (bn >= 128 ? 64 : 32));
   char name[64];
   snprintf(name, sizeof name, "smith_gemm%s_%s_m%u_n%u", g2 ? "2" : "", fmt_tag(fmt), bm, bn);
+  uint32_t threads = 64 * (bm / 64) * (bn / (bn >= 128 ? 64 : 32));
+  // record formats with K % 64 == 0 (dword-aligned records): smith_gemm3_*.
+  // Which shapes the static scratch takes is still decided by the tiles and
+  // splits above.
+  if (g3) {
+    const uint32_t tm = gemm3_plan(fmt, M, N, S, &ks);
+    sps = (S + ks - 1) / ks;
+    if (ks > 1 && ensure(c, (void**)&c->ws, &c->ws_bytes, (size_t)ks * M * N * sizeof(float))) return -1;
+    snprintf(name, sizeof name, "smith_gemm3_%s_m%u", fmt_tag(fmt), tm);
+    tiles = ntiles(16 * tm, 256), threads = 512;
+  }
   const void* pA = c->a16;
   const void* pB = B;
   const void* pD = D;
@@ -711,9 +758,6 @@ struct SmithEncoder {
 //   [64 KiB, +4 MiB)       activation fragments (M > 8 GEMV prep; f16 A of
 //                          the M >= 64 GEMM)
 //   [4 MiB + 64 KiB, 32 MiB)  split-K partials
-constexpr size_t NOALLOC_BYTES = 32u << 20;
-constexpr size_t NOALLOC_CNT_BYTES = 64u << 10;
-constexpr size_t NOALLOC_PREP_BYTES = 4u << 20;
 static __device__ __align__(256) uint8_t scratch[NOALLOC_BYTES];
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static void* g_scratch_dev[NOALLOC_MAX_DEVICES];
