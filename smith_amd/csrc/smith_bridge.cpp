@@ -1263,12 +1263,12 @@ int smith_quantize_q4(void* ctx, const float* w, void* out, uint32_t K, uint32_t
   Ctx* c = (Ctx*)ctx;
   if (!c) return -1;
   if (set_device(c)) return -1;
-  uint64_t total = (uint64_t)((K + 31) / 32) * N;
-  if (!total) return 0;
+  const uint32_t groups = K / 32 + (K % 32 != 0);
+  if (!groups || !N) return 0;
   uint32_t pK = K, pN = N;
   void* args[] = {&w, &out, &pK, &pN};
-  return launch(c, "smith_quantize_q4s", dim3((unsigned)std::min<uint64_t>((total + 255) / 256, 1 << 20)),
-                dim3(256), args);
+  return launch(c, "smith_quantize_q4s", dim3(N / 256 + (N % 256 != 0), std::min<uint32_t>(groups, 65535)), dim3(256),
+                args);
 }
 
 int smith_quantize_q8(void* ctx, const float* w, void* out, uint32_t K, uint32_t N) {
