@@ -343,6 +343,14 @@ int smith_lmhead_q4_0_greedy(void* ctx, const float* x, const float* norm_gamma,
                              int32_t* tokens, int32_t* count, int32_t* pos, void* act_out, const float* gamma_out,
                              const float* rope_cos, const float* rope_sin, uint32_t rope_len, uint32_t wq,
                              uint32_t wk, float* rope_row);
+/* The LM heads above for M rows of x (row length K) at once: y is [M][N], the
+ * logits of a prompt's rows.  f32 accuracy (split f16 operands on the matrix
+ * cores, f32 where a result is not finite); one row runs the single-row
+ * kernel.  Same shape rules as smith_lmhead_q4_0_nb / smith_lmhead_q6_k_nb. */
+int smith_lmhead_q4_0_rows(void* ctx, const float* x, uint32_t M, const float* norm_gamma, float eps, const void* nib,
+                           const void* d, float* y, uint32_t K, uint32_t N);
+int smith_lmhead_q6_k_rows(void* ctx, const float* x, uint32_t M, const float* norm_gamma, float eps,
+                           const void* planes, float* y, uint32_t K, uint32_t N);
 /* f32 GEMV, W [K][N] (w_is_nk = 0) or [N][K] (weight tying, 1). */
 int smith_gemv_f32(void* ctx, const float* x, const float* norm_gamma, float eps, const float* W, float* y,
                    uint32_t K, uint32_t N, int w_is_nk);

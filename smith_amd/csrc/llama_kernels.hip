@@ -1492,6 +1492,336 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 }
 
 // ---------------------------------------------------------------------------
+// LM head of several rows (the logits of a prompt): y[m][n] = sum_k
+// rmsnorm(x)[m][k] * lmHead[k][n] on the planes of the single-row heads, f32
+// accuracy from f16 MFMAs: x and the weights are split into a rounded f16 and
+// the f16 of what is left, and three of the four products are summed in f32
+// (the fourth is below 2^-22 of the result).  A row is scaled by a power of
+// two so that its largest element is in [2^10, 2^11): the second parts are
+// then good to 2^-34 of it.  A Q4_0 weight d * (q - 8) is a whole multiple of
+// 2^-24 (as d is) of at most 15 bits, so its two parts are exact; Q6_K's d *
+// scale * (q - 32) has up to 24 bits, of which the parts hold 22.
+//
+//   smith_lmhead_split_rows: the rows (optional RMSNorm) as MFMA operands,
+//     frag[part][m / 16][k / 32][lane][8]: one contiguous KB a wave and load
+//   smith_lmhead_<q4_0|q6_k>_rows_m<MT>: workgroup = 256 columns x 16*MT rows;
+//     two waves along N of 128 columns, four along K, their sums joined in
+//     LDS.  The planes hold eight outputs of eight rows k to a lane, so lane
+//     (c, kq) of an MFMA takes output octet c and row octet kq, and fragment f
+//     of the eight it forms is output 8c + f: a lane ends with eight
+//     consecutive outputs of a row.
+// An output that is not finite (a weight beyond the f16 range, an infinite or
+// NaN x) is redone in f32 as the single-row heads compute it.
+// Bounded by the MFMAs: per 32 rows k, 24 MT of them (384 MT clocks) beside
+// ~170 (Q4_0) / ~430 (Q6_K) vector instructions.  K = 3072, N = 32000, 128
+// rows: Q4_0 78 us, Q6_K 92 us, where row by row took 128 launches of 18 /
+// 30 us.  Error against 64 bits 1.2e-7 to 1.7e-7 at K = 1024 .. 4096 (the
+// single-row heads 3.3e-7 to 3.8e-7).
+// ---------------------------------------------------------------------------
+typedef _Float16 lh2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ float lmh_pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+
+// one row per workgroup; rows M .. 16 * ceil(M / 16) - 1 are zeros
+extern "C" __global__ __launch_bounds__(256) void smith_lmhead_split_rows(const float* __restrict__ x,
+                                                                         const float* __restrict__ gamma, float eps,
+                                                                         _Float16* __restrict__ frag,
+                                                                         float* __restrict__ rscale, uint32_t M,
+                                                                         uint32_t K) {
+  __shared__ float red[2][4];
+  const uint32_t m = blockIdx.x, tid = threadIdx.x, KP = (K + 31) / 32;
+  const float* xr = x + (size_t)m * K;
+  const bool live = m < M;
+  float v[32], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 32; i++) {
+    const uint32_t k = tid + 256 * i;
+    v[i] = live && k < K ? xr[k] : 0.f;
+    ss = __builtin_fmaf(v[i], v[i], ss);
+  }
+  if (gamma) {
+    ss = sum64_lanes(ss);
+    if ((tid & 63) == 0) red[0][tid >> 6] = ss;
+    __syncthreads();
+    const float rms = 1.0f / __builtin_sqrtf((red[0][0] + red[0][1] + red[0][2] + red[0][3]) / (float)K + eps);
+#pragma unroll
+    for (int i = 0; i < 32; i++) {
+      const uint32_t k = tid + 256 * i;
+      if (k < K) v[i] = v[i] * rms * gamma[k];
+    }
+  }
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < 32; i++) {
+    const float a = __builtin_fabsf(v[i]);
+    mx = a > mx ? a : mx;
+  }
+  mx = max16_lanes(mx);
+  {
+    const float b = __shfl_xor(mx, 16);
+    mx = b > mx ? b : mx;
+    const float c = __shfl_xor(mx, 32);
+    mx = c > mx ? c : mx;
+  }
+  if ((tid & 63) == 0) red[1][tid >> 6] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; w++) mx = red[1][w] > mx ? red[1][w] : mx;
+  // x * 2^up; a zero, tiny or infinite row keeps 2^0 .. 2^96
+  int up = mx > 0.f && mx < __builtin_inff() ? 10 - ((int)(__float_as_uint(mx) >> 23) - 127) : 0;
+  up = up > 96 ? 96 : (up < -96 ? -96 : up);
+  const float sc = lmh_pow2(up);
+  if (tid == 0) rscale[m] = lmh_pow2(-up);
+  const size_t plane = (size_t)gridDim.x * KP * 32;
+  _Float16* f = frag + (size_t)(m / 16) * KP * 512 + (m % 16) * 8;
+#pragma unroll
+  for (int i = 0; i < 32; i++) {
+    const uint32_t k = tid + 256 * i;
+    if (k >= KP * 32) continue;
+    const float a = v[i] * sc;
+    const _Float16 h = (_Float16)a;
+    const size_t o = (size_t)(k / 32) * 512 + (k % 32) / 8 * 128 + k % 8;
+    f[o] = h;
+    f[plane + o] = (_Float16)(a - (float)h);
+  }
+}
+
+// the f32 value of output n of row xr (after the norm), as the single-row
+// heads form it
+template <bool Q6>
+__device__ __forceinline__ float lmh_f32(const float* __restrict__ xr, const float* __restrict__ gamma, float eps,
+                         const uint8_t* __restrict__ nib, const uint8_t* __restrict__ dsc, uint32_t K, uint32_t N,
+                         uint32_t n) {
+  float rms = 1.f, ss = 0.f;
+  if (gamma) {
+    for (uint32_t k = 0; k < K; k++) ss = __builtin_fmaf(xr[k], xr[k], ss);
+    rms = 1.0f / __builtin_sqrtf(ss / (float)K + eps);
+  }
+  size_t ohb = 0, osc = 0, od = 0, tot;
+  if (Q6) lmh6_offsets(K, N, &ohb, &osc, &od, &tot);
+  const uint32_t vb = n / 32, sub = n % 32 / 8, e = n % 8;
+  float acc = 0.f, corr = 0.f;
+  for (uint32_t k = 0; k < K; k++) {
+    const float xv = gamma ? xr[k] * rms * gamma[k] : xr[k];
+    const size_t g = ((size_t)(k / 8) * (N / 32) + vb) * 4 + sub;
+    const uint32_t w = *(const uint32_t*)(nib + g * 32 + (k % 8) * 4);
+    uint32_t q = (w >> (4 * e)) & 15u;
+    float c;
+    if (Q6) {
+      q |= ((*(const uint16_t*)(nib + ohb + g * 16 + (k % 8) * 2) >> (2 * e)) & 3u) << 4;
+      const float d = (float)((const _Float16*)(nib + od))[(size_t)(n / 256) * K + k];
+      c = xv * (d * (float)((const int8_t*)(nib + osc))[(size_t)(n / 16) * K + k]);
+    } else {
+      c = xv * (float)((const _Float16*)dsc)[((size_t)(k / 8) * (N / 32) + vb) * 8 + k % 8];
+    }
+    corr += c;
+    acc = __builtin_fmaf(c, (float)q, acc);
+  }
+  return __builtin_fmaf(Q6 ? -32.0f : -8.0f, corr, acc);
+}
+
+// what a lane reads for eight rows k of its eight outputs
+template <bool Q6>
+struct LmhW {
+  u32x4 n[2], h, d;
+  uint2 sc;
+};
+
+template <bool Q6, int MT>
+__device__ __forceinline__ void lmhead_rows_body(const _Float16* __restrict__ frag, const float* __restrict__ rscale,
+                                                const uint8_t* __restrict__ nib, const uint8_t* __restrict__ dsc,
+                                                float* __restrict__ y, uint32_t M, uint32_t K, uint32_t N,
+                                                const float* __restrict__ x, const float* __restrict__ gamma,
+                                                float eps) {
+  typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+  __shared__ f32x4_t red[4 * MT * 8 * 64];
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t wn = wave & 1, wk = wave >> 1;
+  const uint32_t c = lane & 15, kq = lane >> 4;
+  const uint32_t NB = N / 32, KO = K / 8, KP = (K + 31) / 32;
+  const uint32_t m0 = blockIdx.x * 16 * MT, n0 = blockIdx.y * 256 + wn * 128 + 8 * c;
+  const uint32_t nc = n0 < N ? n0 : N - 8;  // lanes past N read the last outputs and store nothing
+  const uint32_t vb = nc / 32, sub = nc % 32 / 8;
+  const uint32_t per = (KP + 3) / 4, s0 = wk * per < KP ? wk * per : KP, s1 = s0 + per < KP ? s0 + per : KP;
+  const size_t plane = (size_t)((M + 15) / 16) * KP * 512;
+  size_t ohb = 0, osc = 0, od = 0, tot;
+  if (Q6) lmh6_offsets(K, N, &ohb, &osc, &od, &tot);
+
+  auto loadw = [&](uint32_t s) {
+    LmhW<Q6> w;
+    const uint32_t o = 4 * s + kq < KO ? 4 * s + kq : KO - 1;  // x is zero past K
+    const size_t g = ((size_t)o * NB + vb) * 4 + sub;
+    w.n[0] = *(const u32x4*)(nib + g * 32);
+    w.n[1] = *(const u32x4*)(nib + g * 32 + 16);
+    if constexpr (Q6) {
+      w.h = *(const u32x4*)(nib + ohb + g * 16);
+      w.sc = *(const uint2*)(nib + osc + (size_t)(nc / 16) * K + 8 * o);
+      w.d = *(const u32x4*)(nib + od + ((size_t)(nc / 256) * K + 8 * o) * 2);
+    } else {
+      w.d = *(const u32x4*)(dsc + ((size_t)o * NB + vb) * 16);
+    }
+    return w;
+  };
+  auto loada = [&](u32x4 (&a)[MT][2], uint32_t s) {
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      const uint32_t t = m0 / 16 + mt < (M + 15) / 16 ? m0 / 16 + mt : (M + 15) / 16 - 1;
+      const _Float16* p = frag + ((size_t)t * KP + s) * 512 + lane * 8;
+      a[mt][0] = *(const u32x4*)p;
+      a[mt][1] = *(const u32x4*)(p + plane);
+    }
+  };
+
+  f32x4_t acc[MT][8];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int f = 0; f < 8; f++) acc[mt][f] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  uint32_t e1024 = 0x64006400u, e64 = 0x54005400u;  // in registers: one v_and_or a pair
+  asm volatile("" : "+v"(e1024), "+v"(e64));
+  LmhW<Q6> w = {};
+  u32x4 a[MT][2];
+  if (s0 < s1) {
+    w = loadw(s0);
+    loada(a, s0);
+  }
+  for (uint32_t s = s0; s < s1; s++) {
+    const LmhW<Q6> cw = w;
+    u32x4 ca[MT][2];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) ca[mt][0] = a[mt][0], ca[mt][1] = a[mt][1];
+    const uint32_t sn = s + 1 < s1 ? s + 1 : s;
+    w = loadw(sn);
+    loada(a, sn);
+    // scales of the row pairs (k, k+1): Q4_0 d; Q6_K d * scale as a rounded
+    // f16 and the (exact) rest
+    lh2 sh[4], sl[4];
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+      const uint32_t dw = cw.d[p];
+      const lh2 d2 = __builtin_bit_cast(lh2, dw);
+      if constexpr (Q6) {
+        const uint32_t sw = p < 2 ? cw.sc.x : cw.sc.y;
+        const float f0 = (float)d2.x * (float)(int8_t)((sw >> (16 * (p & 1))) & 0xFFu);
+        const float f1 = (float)d2.y * (float)(int8_t)((sw >> (16 * (p & 1) + 8)) & 0xFFu);
+        sh[p] = (lh2){(_Float16)f0, (_Float16)f1};
+        sl[p] = (lh2){(_Float16)(f0 - (float)sh[p].x), (_Float16)(f1 - (float)sh[p].y)};
+      } else {
+        sh[p] = d2;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < 4; b++) {  // outputs 2b and 2b + 1 of the octet
+      u32x4 wh[2], wl[2];
+#pragma unroll
+      for (int p = 0; p < 4; p++) {
+        // byte b of rows 2p and 2p + 1 in the low bytes of the two halves
+        const uint32_t t = __builtin_amdgcn_perm(cw.n[p / 2][2 * (p & 1) + 1], cw.n[p / 2][2 * (p & 1)],
+                                                 0x0C000C00u | (uint32_t)(4 + b) << 16 | (uint32_t)b);
+        uint32_t u[2] = {(t & 0x000F000Fu) | e1024, (t & 0x00F000F0u) | e64};
+        if constexpr (Q6) {
+          const uint32_t H = cw.h[p];
+          u[0] |= (b < 1 ? H << 4 : H >> (4 * b - 4)) & 0x00300030u;
+          u[1] |= (b < 2 ? H << (6 - 4 * b) : H >> (4 * b - 6)) & 0x03000300u;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const _Float16 off = (_Float16)((i ? 64.0f : 1024.0f) + (Q6 ? 32.0f : 8.0f));
+          const lh2 q = __builtin_bit_cast(lh2, u[i]) - (lh2){off, off};  // exact
+          const lh2 hi = q * sh[p];
+          lh2 lo = __builtin_elementwise_fma(q, sh[p], -hi);
+          if constexpr (Q6) lo = __builtin_elementwise_fma(q, sl[p], lo);
+          wh[i][p] = __builtin_bit_cast(uint32_t, hi);
+          wl[i][p] = __builtin_bit_cast(uint32_t, lo);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const half8_t bh = __builtin_bit_cast(half8_t, wh[i]), bl = __builtin_bit_cast(half8_t, wl[i]);
+        // the three products of these 32 rows k from zero, then one rounding
+        // at the size of the running sum (adding each to it took the error
+        // past the single-row heads' from K = 4096: 3.7e-7 for 3.4e-7)
+        f32x4_t t[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+          t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ca[mt][1]), bh,
+                                                         (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+          t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ca[mt][0]), bl, t[mt], 0, 0, 0);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+          t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ca[mt][0]), bh, t[mt], 0, 0, 0);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) acc[mt][2 * b + i] += t[mt];
+      }
+    }
+  }
+
+  // sums over the four K parts: (2 -> 0, 3 -> 1), then (1 -> 0)
+  auto slot = [&](uint32_t z, int mt, int f) -> f32x4_t& { return red[((z * MT + mt) * 8 + f) * 64 + lane]; };
+#pragma unroll
+  for (int round = 0; round < 2; round++) {
+    const uint32_t half = round == 0 ? 2 : 1;
+    if (wk >= half && wk < 2 * half) {
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int f = 0; f < 8; f++) slot(wn * 2 + wk - half, mt, f) = acc[mt][f];
+    }
+    __syncthreads();
+    if (wk < half) {
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int f = 0; f < 8; f++) acc[mt][f] += slot(wn * 2 + wk, mt, f);
+    }
+    __syncthreads();
+  }
+  if (wk != 0 || n0 >= N) return;
+  bool bad = false;
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const uint32_t m = m0 + 16 * mt + 4 * kq + e;
+      if (m >= M) continue;
+      const float rs = rscale[m];
+      float v[8];
+#pragma unroll
+      for (int f = 0; f < 8; f++) {
+        v[f] = acc[mt][f][e] * rs;
+        bad |= !(__builtin_fabsf(v[f]) < __builtin_inff());
+      }
+      float4* o = (float4*)(y + (size_t)m * N + n0);
+      o[0] = make_float4(v[0], v[1], v[2], v[3]);
+      o[1] = make_float4(v[4], v[5], v[6], v[7]);
+    }
+  if (!bad) return;
+#pragma unroll 1
+  for (uint32_t i = 0; i < 32 * MT; i++) {  // this lane's own outputs again
+    const uint32_t m = m0 + 16 * (i / 32) + 4 * kq + i / 8 % 4, n = n0 + i % 8;
+    if (m < M && !(__builtin_fabsf(y[(size_t)m * N + n]) < __builtin_inff()))
+      y[(size_t)m * N + n] = lmh_f32<Q6>(x + (size_t)m * K, gamma, eps, nib, dsc, K, N, n);
+  }
+}
+
+#define DEF_LMHEAD_ROWS(NAME, Q6, MT)                                                                          \
+  extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void NAME(              \
+      const _Float16* __restrict__ frag, const float* __restrict__ rscale, const uint8_t* __restrict__ nib,    \
+      const uint8_t* __restrict__ dsc, float* __restrict__ y, uint32_t M, uint32_t K, uint32_t N,              \
+      const float* __restrict__ x, const float* __restrict__ gamma, float eps) {                               \
+    lmhead_rows_body<Q6, MT>(frag, rscale, nib, dsc, y, M, K, N, x, gamma, eps);                               \
+  }
+DEF_LMHEAD_ROWS(smith_lmhead_q4_0_rows_m1, false, 1)
+DEF_LMHEAD_ROWS(smith_lmhead_q4_0_rows_m2, false, 2)
+DEF_LMHEAD_ROWS(smith_lmhead_q4_0_rows_m4, false, 4)
+DEF_LMHEAD_ROWS(smith_lmhead_q6_k_rows_m1, true, 1)
+DEF_LMHEAD_ROWS(smith_lmhead_q6_k_rows_m2, true, 2)
+DEF_LMHEAD_ROWS(smith_lmhead_q6_k_rows_m4, true, 4)
+
+// ---------------------------------------------------------------------------
 // GGUF weights [out=N rows, in=K] of Q4_0 / Q4_1 / Q5_0 / Q4_K / Q6_K blocks
 // -> the tile planes of gguf_tiles.h.  Values are moved, never changed: the
 // same integers, f16 fields and 6-bit / int8 scales the reference's decoders

@@ -2000,6 +2000,58 @@ int smith_lmhead_q6_k_greedy(void* ctx, const float* x, const float* norm_gamma,
   return lmhead_q6_k(c, "smith_lmhead_q6_k_greedy", x, norm_gamma, eps, planes, logits, K, N, gt);
 }
 
+// logits of M rows: the rows as split f16 operands, then the MFMA kernel.
+// 64 rows a workgroup from 33 rows up (an operand fetched once per 64 rows),
+// else the smallest tile that holds them.
+static int lmhead_rows(Ctx* c, const char* kernel, const float* x, uint32_t M, const float* norm_gamma, float eps,
+                       const void* nib, const void* d, float* y, uint32_t K, uint32_t N) {
+  const uint32_t MT = M <= 16 ? 1 : (M <= 32 ? 2 : 4), M16 = (M + 15) / 16 * 16, KP = (K + 31) / 32;
+  const size_t frag_bytes = (size_t)M16 * KP * 32 * 2 * 2;
+  if (ensure(c, &c->prep, &c->prep_bytes, frag_bytes + M16 * sizeof(float))) return -1;
+  void* frag = c->prep;
+  void* rs = (char*)c->prep + frag_bytes;
+  void* pargs[] = {&x, &norm_gamma, &eps, &frag, &rs, &M, &K};
+  if (launch(c, "smith_lmhead_split_rows", dim3(M16), dim3(256), pargs)) return -1;
+  char name[64];
+  snprintf(name, sizeof name, "%s_m%u", kernel, MT);
+  void* args[] = {&frag, &rs, &nib, &d, &y, &M, &K, &N, &x, &norm_gamma, &eps};
+  return launch(c, name, dim3((M + 16 * MT - 1) / (16 * MT), (N + 255) / 256), dim3(512), args);
+}
+
+int smith_lmhead_q4_0_rows(void* ctx, const float* x, uint32_t M, const float* norm_gamma, float eps, const void* nib,
+                           const void* d, float* y, uint32_t K, uint32_t N) {
+  Ctx* c = (Ctx*)ctx;
+  if (!c) return -1;
+  const char* who = "smith_lmhead_q4_0_rows";
+  if (M <= 1 || ((uintptr_t)y & 15)) {
+    for (uint32_t m = 0; m < M; m++)
+      if (lmhead_q4_0(c, who, x + (size_t)m * K, norm_gamma, eps, nib, d, y + (size_t)m * N, K, N, GreedyTail{}))
+        return -1;
+    return 0;
+  }
+  if (N % 32 || !N) return fail(c, "%s: vocab %u is not a multiple of 32", who, N);
+  if (K > 8192 || K % 8 || !K) return fail(c, "%s: dim %u unsupported (8..8192, %% 8)", who, K);
+  if (set_device(c)) return -1;
+  return lmhead_rows(c, who, x, M, norm_gamma, eps, nib, d, y, K, N);
+}
+
+int smith_lmhead_q6_k_rows(void* ctx, const float* x, uint32_t M, const float* norm_gamma, float eps,
+                           const void* planes, float* y, uint32_t K, uint32_t N) {
+  Ctx* c = (Ctx*)ctx;
+  if (!c) return -1;
+  const char* who = "smith_lmhead_q6_k_rows";
+  if (M <= 1 || ((uintptr_t)y & 15)) {
+    for (uint32_t m = 0; m < M; m++)
+      if (lmhead_q6_k(c, who, x + (size_t)m * K, norm_gamma, eps, planes, y + (size_t)m * N, K, N, GreedyTail{}))
+        return -1;
+    return 0;
+  }
+  if (N % 256 || !N) return fail(c, "%s: vocab %u is not a multiple of 256", who, N);
+  if (K > 8192 || K % 16 || !K) return fail(c, "%s: dim %u unsupported (16..8192, %% 16)", who, K);
+  if (set_device(c)) return -1;
+  return lmhead_rows(c, who, x, M, norm_gamma, eps, planes, nullptr, y, K, N);
+}
+
 int smith_gemv_f32(void* ctx, const float* x, const float* norm_gamma, float eps, const float* W, float* y,
                    uint32_t K, uint32_t N, int w_is_nk) {
   Ctx* c = (Ctx*)ctx;

@@ -111,6 +111,8 @@ SYMBOLS = {
     "smith_lmhead_q4_0_nb": (_INT, [_P, _P, _P, ctypes.c_float, _P, _P, _P, _U32, _U32]),
     "smith_lmhead_q4_0_greedy": (_INT, [_P, _P, _P, ctypes.c_float, _P, _P, _P, _U32, _U32, _P, _P, _P, _P, _P, _P,
                                         _P, _P, _P, _U32, _U32, _U32, _P]),
+    "smith_lmhead_q4_0_rows": (_INT, [_P, _P, _U32, _P, ctypes.c_float, _P, _P, _P, _U32, _U32]),
+    "smith_lmhead_q6_k_rows": (_INT, [_P, _P, _U32, _P, ctypes.c_float, _P, _P, _U32, _U32]),
     "smith_gemv_f32": (_INT, [_P, _P, _P, ctypes.c_float, _P, _P, _U32, _U32, _INT]),
     "smith_argmax_embed": (_INT, [_P, _P, _U32, _P, _U32, _P, _P, _P, _P, _P, _P, _P, _P, _U32, _U32, _U32, _P]),
     "smith_set_i32": (_INT, [_P, _P, ctypes.c_int32]),
@@ -255,6 +257,12 @@ def download(buf, nbytes, dtype, offset=0):
     """Device -> host copy into a new numpy array (waits for the stream)."""
     import numpy as np
     out = np.empty(int(nbytes) // np.dtype(dtype).itemsize, dtype=dtype)
+    check(lib.smith_copy_d2h(ctx(), out.ctypes.data_as(_P), buf, offset, out.nbytes), "smith_copy_d2h")
+    return out
+
+
+def download_into(out, buf, offset=0):
+    """Device -> host copy into a contiguous numpy array (waits for the stream)."""
     check(lib.smith_copy_d2h(ctx(), out.ctypes.data_as(_P), buf, offset, out.nbytes), "smith_copy_d2h")
     return out
 

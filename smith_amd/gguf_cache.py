@@ -74,6 +74,7 @@ class _Engine:
         self.attn = DeviceArray((R, dim))
         self.h = DeviceArray((R, ffn))
         self.logits = DeviceArray((cfg["vocabSize"],))
+        self.row_logits = None  # [rows, vocab] of a prompt's logits, made for the first such call
         self.pos = DeviceArray((1,), np.int32)
         self.count = DeviceArray((1,), np.int32)
         self.tokens = DeviceArray((cfg["maxSeqLen"] + 1,), np.int32)
@@ -166,22 +167,22 @@ class _Engine:
             return None, None
         return self.act_x.ptr, model["blocks"][0]["ln1Gamma"].ptr
 
-    def lm_head(self, model, x_ptr):
+    def lm_head(self, model, x_ptr, out_ptr=None):
         """Final RMSNorm fused into the LM head (gguf_cache.js:174-184)."""
         cfg, ctx = self.cfg, device.ops_ctx()
+        out = self.logits.ptr if out_ptr is None else out_ptr
         head, g, eps = model["lmHead"], model["lnFGamma"].ptr, model["normEps"]
         if head["kind"] == "q4_0_nb":
-            rc = device.lib.smith_lmhead_q4_0_nb(ctx, x_ptr, g, eps, head["nib"].ptr, head["d"].ptr, self.logits.ptr,
-                                                 cfg["dim"],
-                                                 cfg["vocabSize"])
+            rc = device.lib.smith_lmhead_q4_0_nb(ctx, x_ptr, g, eps, head["nib"].ptr, head["d"].ptr, out,
+                                                 cfg["dim"], cfg["vocabSize"])
         elif head["kind"] == "q6_k_nb":
-            rc = device.lib.smith_lmhead_q6_k_nb(ctx, x_ptr, g, eps, head["planes"].ptr, self.logits.ptr, cfg["dim"],
+            rc = device.lib.smith_lmhead_q6_k_nb(ctx, x_ptr, g, eps, head["planes"].ptr, out, cfg["dim"],
                                                  cfg["vocabSize"])
         elif head["kind"] == "f32_kn":
-            rc = device.lib.smith_gemv_f32(ctx, x_ptr, g, eps, head["w"].ptr, self.logits.ptr, cfg["dim"],
+            rc = device.lib.smith_gemv_f32(ctx, x_ptr, g, eps, head["w"].ptr, out, cfg["dim"],
                                            cfg["vocabSize"], 0)
         else:
-            rc = device.lib.smith_gemv_f32(ctx, x_ptr, g, eps, model["embedding"].ptr, self.logits.ptr, cfg["dim"],
+            rc = device.lib.smith_gemv_f32(ctx, x_ptr, g, eps, model["embedding"].ptr, out, cfg["dim"],
                                            cfg["vocabSize"], 1)
         device.check(rc, "lm head")
 
@@ -225,27 +226,49 @@ class _Engine:
         device.check(device.lib.smith_embed(device.ops_ctx(), model["embedding"].ptr, self.tok_in.ptr, self.x.ptr,
                                             len(t), self.cfg["dim"], a0, g0), "embed")
 
+    def lm_head_rows(self, model, M, out_ptr):
+        """lm_head of rows x[0:M] into [M, vocab] at out_ptr: one launch over
+        the rows for a Q4_0 or Q6_K head, else row by row."""
+        cfg, ctx = self.cfg, device.ops_ctx()
+        head, g, eps = model["lmHead"], model["lnFGamma"].ptr, model["normEps"]
+        if head["kind"] == "q4_0_nb":
+            rc = device.lib.smith_lmhead_q4_0_rows(ctx, self.x.ptr, M, g, eps, head["nib"].ptr, head["d"].ptr, out_ptr,
+                                                   cfg["dim"], cfg["vocabSize"])
+            device.check(rc, "lm head")
+        elif head["kind"] == "q6_k_nb":
+            rc = device.lib.smith_lmhead_q6_k_rows(ctx, self.x.ptr, M, g, eps, head["planes"].ptr, out_ptr, cfg["dim"],
+                                                   cfg["vocabSize"])
+            device.check(rc, "lm head")
+        else:
+            for r in range(M):
+                self.lm_head(model, self.x.ptr + r * cfg["dim"] * 4, out_ptr + r * cfg["vocabSize"] * 4)
+
     def prefill(self, model, tokens, caches, all_logits=False):
         """Prompt rows in chunks of <= 256 (attention keeps a chunk's keys in
         LDS); returns the logits of every row if asked, else of the last."""
         n = len(tokens)
-        rows = []
-        step = _chunk_rows(self.cfg)
+        step, dim, vocab = _chunk_rows(self.cfg), self.cfg["dim"], self.cfg["vocabSize"]
+        logits = np.empty((n, vocab), np.float32) if all_logits else None
+        if all_logits and (self.row_logits is None or self.row_logits.shape[0] < min(n, step)):
+            from .gguf_loader import DeviceArray
+            old, self.row_logits = self.row_logits, None
+            if old is not None:
+                device.release_buffer(old.ptr)
+            self.row_logits = DeviceArray((min(n, step), vocab))
         for r0 in range(0, n, step):
             r1 = min(n, r0 + step)
             self.embed(model, tokens[r0:r1])
             self.set_pos(r0)
             self.layers(model, caches, r1 - r0)
             if all_logits:
-                for r in range(r1 - r0):
-                    self.lm_head(model, self.x.ptr + r * self.cfg["dim"] * 4)
-                    rows.append(self.logits.numpy().copy())
+                self.lm_head_rows(model, r1 - r0, self.row_logits.ptr)
+                device.download_into(logits[r0:r1], self.row_logits.ptr)
         last = (n - 1) % step
         if not all_logits:
-            self.lm_head(model, self.x.ptr + last * self.cfg["dim"] * 4)
+            self.lm_head(model, self.x.ptr + last * dim * 4)
         for c in caches:
             c["len"] = n
-        return np.stack(rows) if all_logits else None
+        return logits
 
 
 def _engine(model):
