@@ -47,6 +47,7 @@ struct Ctx {
   std::string err;
   std::vector<Library*> libs;
   Library* ops = nullptr;
+  std::unordered_map<std::string, hipFunction_t> kernels;  // op kernels found so far (find_kernel)
   std::vector<Pipeline*> pipelines;
   uint64_t allocated = 0;
   // op scratch: prepared activations, split-K partials, split-K counters
@@ -157,21 +158,26 @@ hipEvent_t pooled_event(Ctx* c) {
 }
 
 // Op kernels may live in any loaded code object (smith_kernels.hsaco,
-// smith_llama.hsaco, ...): first match in load order wins.
+// smith_llama.hsaco, ...): first match in load order wins.  Found once per
+// name and kept by the context: a lookup that misses in an earlier code object
+// is slow and leaves hipErrorNotFound behind (taken out here, so that another
+// user of the runtime in this thread does not see it), and the kernels of the
+// later objects would pay for it on every launch.
 int find_kernel(Ctx* c, const char* name, hipFunction_t* out) {
+  const auto known = c->kernels.find(name);
+  if (known != c->kernels.end()) {
+    *out = known->second;
+    return 0;
+  }
   if (c->libs.empty()) return fail(c, "smith: no code object loaded (call smith_load_library first)");
   for (Library* lib : c->libs) {
-    auto it = lib->fns.find(name);
-    if (it != lib->fns.end()) {
-      *out = it->second;
-      return 0;
-    }
     hipFunction_t f;
     if (hipModuleGetFunction(&f, lib->mod, name) == hipSuccess) {
-      lib->fns[name] = f;
+      c->kernels[name] = f;
       *out = f;
       return 0;
     }
+    (void)hipGetLastError();
   }
   return fail(c, "smith: kernel '%s' not found in any loaded code object", name);
 }
