@@ -8,8 +8,7 @@
 //                       q50t, q4kt, q6kt}
 //   smith_gemm_prep_a_perm + smith_gemm2_<fmt>_m<BM>_n<BN>  the DMA-staged
 //                       GEMM for the tile-plane formats (further below)
-//   smith_gemm3_<fmt>_m<TM>  the DMA-staged GEMM for the record formats (q4s,
-//                       q8, q40) with K % 64 == 0
+//   smith_gemm3_<fmt>_m<TM>  the DMA-staged GEMM of every format, K % 64 == 0
 //
 // Workgroup tile BM x BN (128x64 .. 256x256), K in stages of BK=64 (two
 // 32-row quantization groups), double-buffered in LDS: while the MFMAs
@@ -714,12 +713,14 @@ DEF_GEMM2_FMT(q4kt, GT_Q4K)
 DEF_GEMM2_FMT(q6kt, GT_Q6K)
 
 // ---------------------------------------------------------------------------
-// gemm3: the GEMM on (g, n) records (Q4S, Q8, Q4_0 planes), K % 64 == 0.
+// gemm3: the GEMM on (g, n) records (Q4S, Q8, Q4_0 planes) and on the GGUF
+// tile planes, K % 64 == 0.
 // Workgroup tile 16*TM rows x 256 columns, eight waves side by side along N,
 // each over all the rows and 32 columns.  Stages of K = 64 in a ring of three
 // LDS buffers filled by 16-byte direct-to-LDS loads: the A rows (16-byte
 // chunks XOR-swizzled by row through each lane's source address) and the two
-// groups' raw records, which are contiguous over the tile's columns.  A wave
+// groups' raw records, which are contiguous over the tile's columns (of the
+// tile planes, a contiguous run of each plane per 16 columns).  A wave
 // converts the records of its own columns to f16 in registers beside its
 // MFMAs, so a weight is converted once per workgroup and never written back
 // to LDS.  The MFMA takes the weights as its A operand: a lane then holds four
@@ -734,7 +735,10 @@ DEF_GEMM2_FMT(q6kt, GT_Q6K)
 // 50.1); four waves of 256 x 64 spill.
 // Measured (whole call: activation prep, GEMM, K-split reduce; the register-
 // staged kernel before it): Q4S M = 512, 14336 x 4096 80 -> 66 us; M = 2048,
-// 4096 x 14336 259 -> 242 us; Q8 M = 301, 14336 x 4096 84 -> 57 us.
+// 4096 x 14336 259 -> 242 us; Q8 M = 301, 14336 x 4096 84 -> 57 us; against
+// smith_gemm2_*: Q4_K 28672 x 4096 at 2 / 128 / 250 rows 115 -> 29, 119 -> 53,
+// 121 -> 79 us, Q6_K 4096 x 14336 42 -> 25, 49 -> 42, 74 -> 62 us, Q4_0 18432
+// x 3072 at 250 rows 76 -> 45 us.
 // ---------------------------------------------------------------------------
 // 16 bytes per lane from base + off (a lane's own) to LDS byte address lds +
 // 16 * lane (wave-uniform).  In asm so that the compiler does not see an LDS
@@ -761,14 +765,20 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
 
 template <int FMT, int TM>
 struct G3 {
+  using GF = GtFmt<FMT>;
   static constexpr int NW = 8, TN = 2, BM = 16 * TM, BN = 16 * TN * NW;
+  static constexpr bool TILES = GF::TILES;                                 // tile planes, else (g, n) records
   static constexpr int R = FMT == WF_Q4S ? 24 : (FMT == WF_Q8 ? 34 : 16);  // bytes of a record in B
   static constexpr bool HAS_D = FMT == WF_Q40;
   static constexpr int A_CH = BM / 8;  // 1 KB chunks: 8 rows of 128 B
-  // records of one group, plus up to 3 bytes below a 4-byte aligned start
-  static constexpr int RCH = (BN * R + (R % 4 ? 3 : 0) + 1023) / 1024, RUN = RCH * 1024;
+  // (g, n) records: those of one group, plus up to 3 bytes below a 4-byte
+  // aligned start; tile planes: both groups' nibbles, high bits, parameters
+  // and super-block parameters of the 16 column tiles, each plane a run
+  static constexpr int RCH = TILES ? BN * 32 / 1024 : (BN * R + (R % 4 ? 3 : 0) + 1023) / 1024, RUN = RCH * 1024;
   static constexpr int DCH = HAS_D ? 1 : 0;  // BN f16 scales of one group
-  static constexpr int B_CH = 2 * (RCH + DCH);
+  static constexpr int HCH = TILES ? BN * 2 * GF::HB / 1024 : 0, PCH = TILES ? BN * 2 * GF::PRM / 1024 : 0;
+  static constexpr int SCH = TILES && GF::SUP ? 1 : 0;
+  static constexpr int B_CH = TILES ? RCH + HCH + PCH + SCH : 2 * (RCH + DCH);
   static constexpr int A_PW = (A_CH + NW - 1) / NW, B_PW = (B_CH + NW - 1) / NW, CNT = A_PW + B_PW;  // loads per wave and stage
   static constexpr int STAGE = (A_CH + B_CH) * 1024;
   static_assert(BN * 2 + 3 <= 1024, "one chunk of scales");
@@ -799,7 +809,60 @@ template <int FMT>
 struct G3Raw {
   uint32_t x[FMT == WF_Q8 ? 3 : 1];
   float s, z;
+  uint32_t h, p, sp;  // tile planes: high bits (the word of this K slice), prm, sup
 };
+
+// Tile-plane weights 8 kq .. 8 kq + 7 of a record (gguf_tiles.h), in f16 in
+// the slot order {0,4,1,5,2,6,3,7}: w = s*q + c with q exact
+template <int F>
+__device__ __forceinline__ half8 gt_weight(uint32_t x, uint32_t W, uint32_t prm, uint32_t sup, uint32_t kq,
+                                           uint32_t e1024, uint32_t e64) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  const uint32_t y = x >> 8;
+  uint32_t b0 = (x & 0x000F000Fu) | e1024, b1 = (x & 0x00F000F0u) | e64;
+  uint32_t b2 = (y & 0x000F000Fu) | e1024, b3 = (y & 0x00F000F0u) | e64;
+  if constexpr (F == GT_Q50) {
+    // element 8kq + k: bit 4kq + (k & 3) + 16 (k >> 2)
+    b0 |= ((W >> (4 * kq)) << 4) & 0x00100010u;
+    b1 |= ((W >> (4 * kq + 1)) << 8) & 0x01000100u;
+    b2 |= ((W >> (4 * kq + 2)) << 4) & 0x00100010u;
+    b3 |= ((W >> (4 * kq + 3)) << 8) & 0x01000100u;
+  } else if constexpr (F == GT_Q6K) {
+    const uint32_t cb = 4 * (kq & 1);
+    b0 |= ((W >> (2 * cb)) << 4) & 0x00300030u;
+    b1 |= ((W >> (2 * cb + 2)) << 8) & 0x03000300u;
+    b2 |= ((W >> (2 * cb + 4)) << 4) & 0x00300030u;
+    b3 |= ((W >> (2 * cb + 6)) << 8) & 0x03000300u;
+  }
+  h2 sv, cv;
+  if constexpr (F == GT_Q40 || F == GT_Q50) {
+    const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)prm);
+    const _Float16 c = d * (_Float16)(F == GT_Q40 ? -8.0f : -16.0f);  // exact
+    sv = (h2){d, d};
+    cv = (h2){c, c};
+  } else if constexpr (F == GT_Q41) {
+    const h2 dm = __builtin_bit_cast(h2, prm);  // (d, m)
+    sv = (h2){dm.x, dm.x};
+    cv = (h2){dm.y, dm.y};
+  } else {  // Q4_K, Q6_K: f32 products of the f16 and the 6-bit / int8 scales, rounded to f16
+    float s0f, c0f, s1f, c1f;
+    GtW<F> w;
+    w.p = prm;
+    w.sp = sup;
+    gt_affine<F>(w, s0f, c0f, s1f, c1f);
+    const float sf = kq < 2 ? s0f : s1f, cf = kq < 2 ? c0f : c1f;
+    sv = (h2){(_Float16)sf, (_Float16)sf};
+    cv = (h2){(_Float16)cf, (_Float16)cf};
+  }
+  const h2 blo = (h2){(_Float16)1024.0f, (_Float16)1024.0f}, bhi = (h2){(_Float16)64.0f, (_Float16)64.0f};
+  const h2 v0 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b0) - blo, sv, cv);
+  const h2 v1 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b1) - bhi, sv, cv);
+  const h2 v2 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b2) - blo, sv, cv);
+  const h2 v3 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b3) - bhi, sv, cv);
+  const u32x4 u = {__builtin_bit_cast(uint32_t, v0), __builtin_bit_cast(uint32_t, v1),
+                   __builtin_bit_cast(uint32_t, v2), __builtin_bit_cast(uint32_t, v3)};
+  return __builtin_bit_cast(half8, u);
+}
 
 template <int FMT, int TM>
 __device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, const uint8_t* __restrict__ B,
@@ -832,6 +895,7 @@ __device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, con
   uint32_t lb[P::B_PW];
   const uint8_t* pb[P::B_PW];
   size_t strb[P::B_PW];
+  bool sup[P::B_PW] = {};  // a super-block plane: 8 groups to a stride
   const uint8_t* pa = (const uint8_t*)(A16 + (size_t)m0 * K + (size_t)s0 * 64);
 #pragma unroll
   for (int i = 0; i < P::A_PW; i++) {
@@ -851,6 +915,33 @@ __device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, con
 #pragma unroll
   for (int i = 0; i < P::B_PW; i++) {
     const uint32_t j = wave + P::NW * i < (uint32_t)P::B_CH ? wave + P::NW * i : (uint32_t)P::B_CH - 1;
+    lb[i] = j * 1024;
+    if constexpr (P::TILES) {
+      // chunk j of a plane whose tiles hold tb bytes a stage, tiles apart by ts
+      using GF = typename P::GF;
+      const GtPlanes PL = gt_planes(GF::F, N, K / 32);
+      const uint8_t* prp = FMT == WF_Q40T ? (const uint8_t*)D : B + PL.prm;
+      const uint32_t G = K / 32, tiles = N / 16 - n0 / 16;
+      uint32_t jj, tb, sb;
+      size_t ts;
+      const uint8_t* base;
+      sup[i] = false;
+      if (j < (uint32_t)P::RCH) jj = j, tb = 512, ts = (size_t)G * 256, base = B;
+      else if (j < (uint32_t)(P::RCH + P::HCH)) jj = j - P::RCH, tb = 32 * GF::HB, ts = (size_t)G * 16 * GF::HB, base = B + PL.hb;
+      else if (j < (uint32_t)(P::RCH + P::HCH + P::PCH))
+        jj = j - P::RCH - P::HCH, tb = 32 * GF::PRM, ts = (size_t)G * 16 * GF::PRM, base = prp;
+      else jj = 0, tb = 16 * GF::SUP, ts = (size_t)(G / 8) * 16 * GF::SUP, base = B + PL.sup, sup[i] = true;
+      sb = sup[i] ? 0 : tb;
+      const uint32_t off = jj * 1024 + lane * 16;
+      uint32_t tile = off / (tb ? tb : 16);
+      const uint32_t within = off % (tb ? tb : 16);
+      tile = tile < 16 ? tile : 15;  // a short run: the last tile again
+      tile = tile < tiles ? tile : tiles - 1;
+      vb[i] = (uint32_t)(tile * ts) + within;
+      pb[i] = (const uint8_t*)uniform64((size_t)(base + (size_t)(n0 / 16) * ts + (size_t)s0 * sb));
+      strb[i] = uniform64(sb);
+      continue;
+    }
     const bool isd = P::HAS_D && j >= 2 * P::RCH;
     const uint32_t gi = isd ? j - 2 * P::RCH : j / P::RCH;
     const uint32_t rec = isd ? 2u : (uint32_t)P::R, sh = isd ? (gi ? shd[1] : shd[0]) : (gi ? shq[1] : shq[0]);
@@ -859,7 +950,6 @@ __device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, con
     vb[i] = off < last ? off : last;
     pb[i] = (const uint8_t*)uniform64((size_t)(isd ? (const uint8_t*)D : B) + ((size_t)(2 * s0 + gi) * N + n0) * rec - sh);
     strb[i] = uniform64((size_t)2 * N * rec);
-    lb[i] = j * 1024;
   }
   const uint32_t lds0 = (uint32_t)(size_t)(lds_ptr_t)ring;
   auto issue = [&](uint32_t s, uint32_t buf) {  // stage s0 + s into the buffer at byte buf of the ring
@@ -869,7 +959,11 @@ __device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, con
       dma16(pa + (size_t)s * 128, va[i], lds0 + buf + j * 1024);
     }
 #pragma unroll
-    for (int i = 0; i < P::B_PW; i++) dma16(pb[i] + s * strb[i], vb[i], lds0 + buf + P::A_CH * 1024 + lb[i]);
+    for (int i = 0; i < P::B_PW; i++) {
+      size_t o = s * strb[i];
+      if constexpr (P::SCH) o = sup[i] ? (size_t)((s0 + s) / 4) * 16 * P::GF::SUP : o;
+      dma16(pb[i] + o, vb[i], lds0 + buf + P::A_CH * 1024 + lb[i]);
+    }
   };
 
   f32x4 acc[TM][TN];
@@ -888,7 +982,20 @@ __device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, con
   auto raw = [&](const uint8_t* bs, int j, int kk) {
     G3Raw<FMT> w;
     const uint32_t col = bcol + 16 * j;
-    if constexpr (FMT == WF_Q8) {
+    if constexpr (P::TILES) {
+      using GF = typename P::GF;
+      const uint32_t ri = (col / 16 * 2 + kk) * 16 + col % 16;  // record within the stage
+      w.x[0] = *(const uint32_t*)(bs + ri * 16 + 4 * kq);
+      const uint8_t* p = bs + P::RUN;
+      if constexpr (GF::F == GT_Q50) w.h = *(const uint32_t*)(p + ri * 4);
+      if constexpr (GF::F == GT_Q6K) w.h = *(const uint32_t*)(p + ri * 8 + 4 * (kq >> 1));
+      p += P::HCH * 1024;
+      if constexpr (GF::PRM == 4) w.p = *(const uint32_t*)(p + ri * 4);
+      else w.p = *(const uint16_t*)(p + ri * 2);
+      p += P::PCH * 1024;
+      if constexpr (GF::SUP == 4) w.sp = *(const uint32_t*)(p + col * 4);
+      if constexpr (GF::SUP == 2) w.sp = *(const uint16_t*)(p + col * 2);
+    } else if constexpr (FMT == WF_Q8) {
       const uint32_t o = kk * P::RUN + shq[kk] + col * 34;
       const uint32_t* p = (const uint32_t*)(bs + ((o + 2 + 8 * kq) & ~3u));
       w.x[0] = p[0];
@@ -909,7 +1016,9 @@ __device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, con
     return w;
   };
   auto weight = [&](const G3Raw<FMT>& w, int j, int kk) -> half8 {
-    if constexpr (FMT == WF_Q8) {
+    if constexpr (P::TILES) {
+      return gt_weight<P::GF::F>(w.x[0], w.h, w.p, w.sp, kq, e1024, e64);
+    } else if constexpr (FMT == WF_Q8) {
       const uint32_t a = (shq[kk] + (bcol + 16 * j) * 34 + 2) & 3u;
       const uint32_t x0 = __builtin_amdgcn_alignbyte(w.x[1], w.x[0], a) ^ 0x80808080u;
       const uint32_t x1 = __builtin_amdgcn_alignbyte(w.x[2], w.x[1], a) ^ 0x80808080u;
@@ -1062,6 +1171,14 @@ __device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, con
 DEF_GEMM3_FMT(q4s, WF_Q4S)
 DEF_GEMM3_FMT(q8, WF_Q8)
 DEF_GEMM3_FMT(q40, WF_Q40)
+#define DEF_GEMM3_TILES(TAG, FMT) \
+  DEF_GEMM3(TAG, FMT, 2)          \
+  DEF_GEMM3_FMT(TAG, FMT)
+DEF_GEMM3_TILES(q40t, WF_Q40T)
+DEF_GEMM3_TILES(q41t, GT_Q41)
+DEF_GEMM3_TILES(q50t, GT_Q50)
+DEF_GEMM3_TILES(q4kt, GT_Q4K)
+DEF_GEMM3_TILES(q6kt, GT_Q6K)
 
 template <bool PERM>
 __device__ __forceinline__ void prep_a_row(const float* __restrict__ A, const float* __restrict__ gamma, float eps,

@@ -546,19 +546,21 @@ constexpr size_t NOALLOC_PREP_BYTES = 4u << 20;
 
 // Row tiles per workgroup (TM) and K splits of smith_gemm3_*: the pair with
 // the least estimated time.  256 workgroups run at once (one a CU); a stage
-// of K = 64 takes about 0.35 + 0.076 TM us (Q8, whose conversion is longer,
-// 0.45), filling the ring and storing the tile 3 + 0.35 TM us, and splits add
-// the reduce: partials read and result written at 7.2 TB/s, and 5 us.
+// of K = 64 takes about 0.35 + 0.076 TM us (0.45 for the formats with a longer
+// conversion: Q8, Q4_1 and on), filling the ring and storing the tile 3 + 0.35 TM us, and splits add
+// the reduce: partials read and result written at 7.2 TB/s, and 5 us (fused:
+// it also prepares the next GEMM's rows, a launch less there, and 0.5 us).
 // (Measured on either side: Q4S M = 512, 14336 x 4096 TM = 8 without splits
 // 71 us, 16 with two 81; Q8 M = 301 10 with two 61, 8 without 69; Q4S M =
 // 2048, 4096 x 14336 both 252.)
-uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, uint32_t* ks_out) {
-  const double conv = fmt == FQ8 ? 0.45 : 0.35;
-  static const uint32_t tms[] = {4, 6, 8, 10, 12, 14, 16};
+uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, bool fused, uint32_t* ks_out) {
+  const double conv = fmt == FQ8 || fmt > FQ40T ? 0.45 : 0.35;
+  static const uint32_t tms[] = {2, 4, 6, 8, 10, 12, 14, 16};
   double best = 1e30;
   uint32_t btm = 16;
   *ks_out = 1;
   for (uint32_t tm : tms) {
+    if (tm == 2 && M > 32) continue;  // a weight is converted once per row tile
     const uint64_t tiles = (uint64_t)((M + 16 * tm - 1) / (16 * tm)) * ((N + 255) / 256);
     for (uint32_t ks = 1; ks <= 16 && (ks == 1 || S / ks >= 4); ks++) {
       const uint32_t sps = (S + ks - 1) / ks;
@@ -569,7 +571,7 @@ uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, uint32_t* ks_ou
           (size_t)ks * M * N * sizeof(float) > NOALLOC_BYTES - NOALLOC_CNT_BYTES - NOALLOC_PREP_BYTES)
         break;
       double t = (double)((tiles * ks + 255) / 256) * (sps * (conv + 0.076 * tm) + 3.0 + 0.35 * tm);
-      if (ks > 1) t += 5.0 + (ks + 1.0) * M * N * 4.0 / 7.2e6;
+      if (ks > 1) t += (fused ? 0.5 : 5.0) + (ks + 1.0) * M * N * 4.0 / 7.2e6;
       if (t < best) best = t, btm = tm, *ks_out = ks;
     }
   }
@@ -597,8 +599,15 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
     return !(e && e[0] == '0');
   }();
   const bool g2 = gemm2_on && (fmt == FQ40T || fmt >= FQ41T) && K % 64 == 0;
-  const bool g3 = (fmt == FQ4S || fmt == FQ8 || fmt == FQ40) && K % 64 == 0 &&
-                  ((uintptr_t)B & (fmt == FQ8 ? 1 : 3)) == 0 && ((uintptr_t)D & 1) == 0;
+  // K % 64 == 0: smith_gemm3_* (dword-aligned records and planes; the scales
+  // of Q4_0 records may start at any f16).  Q4_K / Q6_K tiles of 65 .. 128
+  // rows and fewer than 8192 columns keep smith_gemm2_*, whose 64-column
+  // tiles need fewer K splits there (whole calls, 128 rows, gemm2 / gemm3:
+  // Q6_K 3072 x 9216 31.9 / 32.9 us, Q4_K 3072 x 3072 22.2 / 22.4; against
+  // Q4_K 18432 x 3072 41.4 / 36.7, and 3072 x 3072 at 64 rows 17.7 / 16.4).
+  const bool k128 = g2 && (fmt == FQ4KT || fmt == FQ6KT) && M > 64 && M <= 128 && N < 8192;
+  const bool g3 = K % 64 == 0 && !k128 && ((uintptr_t)B & (fmt == FQ8 ? 1 : 3)) == 0 &&
+                  ((uintptr_t)D & (fmt == FQ40 ? 1 : 3)) == 0;
   {
     const float* pa = a;
     const float* pg = ep.gamma;
@@ -608,7 +617,7 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
     void* args[] = {&pa, &pg, &pe, &pd, &pK};
     // the DMA-staged kernels and the register-staged Q4S / Q4_0 ones take A
     // in the permuted slot order of their packed-f16 weight conversion
-    const bool perm = g2 || fmt == FQ4S || fmt == FQ40 || fmt == FQ40T;
+    const bool perm = g2 || (g3 && fmt != FQ8) || fmt == FQ4S || fmt == FQ40 || fmt == FQ40T;
     if (!(pre && perm) && launch(c, perm ? "smith_gemm_prep_a_perm" : "smith_gemm_prep_a", dim3(M), dim3(256), args))
       return -1;
   }
@@ -644,11 +653,10 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
   char name[64];
   snprintf(name, sizeof name, "smith_gemm%s_%s_m%u_n%u", g2 ? "2" : "", fmt_tag(fmt), bm, bn);
   uint32_t threads = 64 * (bm / 64) * (bn / (bn >= 128 ? 64 : 32));
-  // record formats with K % 64 == 0 (dword-aligned records): smith_gemm3_*.
   // Which shapes the static scratch takes is still decided by the tiles and
   // splits above.
   if (g3) {
-    const uint32_t tm = gemm3_plan(fmt, M, N, S, &ks);
+    const uint32_t tm = gemm3_plan(fmt, M, N, S, want_next && ep.mode != 0, &ks);
     sps = (S + ks - 1) / ks;
     if (ks > 1 && ensure(c, (void**)&c->ws, &c->ws_bytes, (size_t)ks * M * N * sizeof(float))) return -1;
     snprintf(name, sizeof name, "smith_gemm3_%s_m%u", fmt_tag(fmt), tm);

@@ -88,3 +88,31 @@ def test_gemm3_epilogues(fmt, epi, M, N, K):
     assert rel2(out.data, y) <= (BAR if epi == 1 else 2 * BAR)
     for b in bufs:
         device.release_buffer(b)
+
+
+# tile planes: row tiles from 32 rows, tiles past the last column, one to a few
+# stages, rows on either side of the 65 .. 128 that Q4_K / Q6_K leave to gemm2
+@pytest.mark.parametrize("t", [O.GGML_Q4_0, O.GGML_Q4_1, O.GGML_Q5_0, O.GGML_Q4_K, O.GGML_Q6_K])
+@pytest.mark.parametrize("M,N,K", [(2, 16, 256), (33, 272, 512), (64, 528, 768), (129, 48, 2048), (200, 1040, 256),
+                                   (257, 8208, 256)])
+def test_gemm3_tiles(t, M, N, K):
+    if t == O.GGML_Q4_0 and M < 64:
+        M = 64  # fewer rows of Q4_0 tiles run the GEMVs
+    w = prng.randn((N, K), 711, std=0.02)
+    blocks = O.quantize_rows(t, w)
+    wd = O.dequantize_tensor(t, blocks, N * K).reshape(N, K).astype(np.float64)
+    L, ctx = device.lib, device.ops_ctx()
+    src, pl = device.alloc(blocks.size), device.alloc(int(L.smith_gguf_tiles_bytes(t, N, K)))
+    device.upload(src, blocks)
+    device.check(L.smith_repack_gguf_tiles_into(ctx, t, src, pl, N, K, 0, 1, N))
+    x = prng.randn((M, K), 712)
+    xt, out = S.tensor(x), S.create([M, N])
+    device.profile_kernels(True)
+    device.check(L.smith_linear_gguf_tiles(ctx, t, xt.buffer, pl, out.buffer, M, N, K, None, 0.0, None, 0))
+    _, n = device.profile_read("smith_gemm3_")
+    device.profile_read("")
+    device.profile_kernels(False)
+    assert n == 1
+    assert rel2(out.data, x.astype(np.float64) @ wd.T) <= BAR
+    for b in (src, pl):
+        device.release_buffer(b)
