@@ -745,7 +745,9 @@ DEF_GEMM2_FMT(q6kt, GT_Q6K)
 // write: it would wait for every load in flight before the next LDS read.
 // There is no destination register, and the kernel counts the loads itself
 // (s_waitcnt vmcnt before the barrier that publishes a stage).  One wait
-// state between the write of M0 and its use.
+// state between the write of M0 and its use.  The compiler warns that M0 is
+// reserved: it must not keep a value there across this, and the emitted code
+// of the kernels that call it uses M0 nowhere else.
 __device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint32_t lds) {
   asm volatile(
       "s_mov_b32 m0, %0\n\t"
