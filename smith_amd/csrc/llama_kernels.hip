@@ -1495,12 +1495,14 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 // LM head of several rows (the logits of a prompt): y[m][n] = sum_k
 // rmsnorm(x)[m][k] * lmHead[k][n] on the planes of the single-row heads, f32
 // accuracy from f16 MFMAs: x and the weights are split into a rounded f16 and
-// the f16 of what is left, and three of the four products are summed in f32
-// (the fourth is below 2^-22 of the result).  A row is scaled by a power of
-// two so that its largest element is in [2^10, 2^11): the second parts are
-// then good to 2^-34 of it.  A Q4_0 weight d * (q - 8) is a whole multiple of
-// 2^-24 (as d is) of at most 15 bits, so its two parts are exact; Q6_K's d *
-// scale * (q - 32) has up to 24 bits, of which the parts hold 22.
+// the f16 of what is left, and all four products are summed in f32.  A row is
+// scaled by a power of two so that its largest element is in [2^14, 2^15), and
+// its second part by another 2^12 (those products are summed apart and come
+// down by 2^12 once per 32 rows k): an element keeps 22 bits down to 2^-28 of
+// the row's largest and is good to 2^-52 of it below that.  A Q4_0 weight
+// d * (q - 8) is a whole multiple of 2^-24 (as d is) of at most 15 bits, so
+// its two parts are exact; Q6_K's d * scale * (q - 32) has up to 24 bits, of
+// which the parts hold 22.
 //
 //   smith_lmhead_split_rows: the rows (optional RMSNorm) as MFMA operands,
 //     frag[part][m / 16][k / 32][lane][8]: one contiguous KB a wave and load
@@ -1512,21 +1514,24 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 //     consecutive outputs of a row.
 // An output that is not finite (a weight beyond the f16 range, an infinite or
 // NaN x) is redone in f32 as the single-row heads compute it.
-// Bounded by the MFMAs: per 32 rows k, 24 MT of them (384 MT clocks) beside
+// Bounded by the MFMAs: per 32 rows k, 32 MT of them (512 MT clocks) beside
 // ~170 (Q4_0) / ~430 (Q6_K) vector instructions.  K = 3072, N = 32000, 128
-// rows: Q4_0 78 us, Q6_K 92 us, where row by row took 128 launches of 18 /
-// 30 us.  Error against 64 bits 1.2e-7 to 1.7e-7 at K = 1024 .. 4096 (the
-// single-row heads 3.3e-7 to 3.8e-7).
+// rows: Q4_0 103 us, Q6_K 113 us, where row by row took 128 launches of 18 /
+// 30 us.  Without the product of the two second parts 85 / 96 us, but rows of
+// a few elements were then less exact than the single-row heads make them
+// (one element, Q6_K: 9.5e-8 for 5.8e-8).  Error against 64 bits 1.0e-7 to
+// 2.0e-7 at K = 1024 .. 8192 (the single-row heads 3.2e-7 to 3.8e-7).
 // ---------------------------------------------------------------------------
 typedef _Float16 lh2 __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ float lmh_pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+#define LMH_LO 12  // log2 of the second part's extra scale
 
-// one row per workgroup; rows M .. 16 * ceil(M / 16) - 1 are zeros
+// one row per workgroup, its logits' exponent in rexp; rows M ..
+// 16 * ceil(M / 16) - 1 are zeros
 extern "C" __global__ __launch_bounds__(256) void smith_lmhead_split_rows(const float* __restrict__ x,
                                                                          const float* __restrict__ gamma, float eps,
                                                                          _Float16* __restrict__ frag,
-                                                                         float* __restrict__ rscale, uint32_t M,
+                                                                         int32_t* __restrict__ rexp, uint32_t M,
                                                                          uint32_t K) {
   __shared__ float red[2][4];
   const uint32_t m = blockIdx.x, tid = threadIdx.x, KP = (K + 31) / 32;
@@ -1567,22 +1572,21 @@ extern "C" __global__ __launch_bounds__(256) void smith_lmhead_split_rows(const 
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < 4; w++) mx = red[1][w] > mx ? red[1][w] : mx;
-  // x * 2^up; a zero, tiny or infinite row keeps 2^0 .. 2^96
-  int up = mx > 0.f && mx < __builtin_inff() ? 10 - ((int)(__float_as_uint(mx) >> 23) - 127) : 0;
-  up = up > 96 ? 96 : (up < -96 ? -96 : up);
-  const float sc = lmh_pow2(up);
-  if (tid == 0) rscale[m] = lmh_pow2(-up);
+  // x * 2^up (up to 2^163, a subnormal row's: not an f32 factor); a zero or
+  // infinite row as it is
+  const int up = mx > 0.f && mx < __builtin_inff() ? 15 - __builtin_amdgcn_frexp_expf(mx) : 0;
+  if (tid == 0) rexp[m] = -up;
   const size_t plane = (size_t)gridDim.x * KP * 32;
   _Float16* f = frag + (size_t)(m / 16) * KP * 512 + (m % 16) * 8;
 #pragma unroll
   for (int i = 0; i < 32; i++) {
     const uint32_t k = tid + 256 * i;
     if (k >= KP * 32) continue;
-    const float a = v[i] * sc;
+    const float a = __builtin_ldexpf(v[i], up);
     const _Float16 h = (_Float16)a;
     const size_t o = (size_t)(k / 32) * 512 + (k % 32) / 8 * 128 + k % 8;
     f[o] = h;
-    f[plane + o] = (_Float16)(a - (float)h);
+    f[plane + o] = (_Float16)((a - (float)h) * (float)(1 << LMH_LO));
   }
 }
 
@@ -1628,7 +1632,7 @@ struct LmhW {
 };
 
 template <bool Q6, int MT>
-__device__ __forceinline__ void lmhead_rows_body(const _Float16* __restrict__ frag, const float* __restrict__ rscale,
+__device__ __forceinline__ void lmhead_rows_body(const _Float16* __restrict__ frag, const int32_t* __restrict__ rexp,
                                                 const uint8_t* __restrict__ nib, const uint8_t* __restrict__ dsc,
                                                 float* __restrict__ y, uint32_t M, uint32_t K, uint32_t N,
                                                 const float* __restrict__ x, const float* __restrict__ gamma,
@@ -1739,22 +1743,26 @@ __device__ __forceinline__ void lmhead_rows_body(const _Float16* __restrict__ fr
 #pragma unroll
       for (int i = 0; i < 2; i++) {
         const half8_t bh = __builtin_bit_cast(half8_t, wh[i]), bl = __builtin_bit_cast(half8_t, wl[i]);
-        // the three products of these 32 rows k from zero, then one rounding
-        // at the size of the running sum (adding each to it took the error
-        // past the single-row heads' from K = 4096: 3.7e-7 for 3.4e-7)
-        f32x4_t t[MT];
+        // the products of these 32 rows k from zero, then one rounding at
+        // the size of the running sum (adding each to it took the error past
+        // the single-row heads' from K = 4096: 3.7e-7 for 3.4e-7)
+        const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+        f32x4_t t[MT][2];
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
-          t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ca[mt][1]), bh,
-                                                         (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+          for (int z = 0; z < 2; z++)
+            t[mt][z] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ca[mt][z]), bl, zero, 0, 0, 0);
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
-          t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ca[mt][0]), bl, t[mt], 0, 0, 0);
+#pragma unroll
+          for (int z = 0; z < 2; z++)
+            t[mt][z] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ca[mt][z]), bh, t[mt][z], 0, 0, 0);
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
-          t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ca[mt][0]), bh, t[mt], 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) acc[mt][2 * b + i] += t[mt];
+          for (int e = 0; e < 4; e++)
+            acc[mt][2 * b + i][e] += __builtin_fmaf(t[mt][1][e], 1.0f / (1 << LMH_LO), t[mt][0][e]);
       }
     }
   }
@@ -1787,11 +1795,11 @@ __device__ __forceinline__ void lmhead_rows_body(const _Float16* __restrict__ fr
     for (int e = 0; e < 4; e++) {
       const uint32_t m = m0 + 16 * mt + 4 * kq + e;
       if (m >= M) continue;
-      const float rs = rscale[m];
+      const int re = rexp[m];
       float v[8];
 #pragma unroll
       for (int f = 0; f < 8; f++) {
-        v[f] = acc[mt][f][e] * rs;
+        v[f] = __builtin_ldexpf(acc[mt][f][e], re);
         bad |= !(__builtin_fabsf(v[f]) < __builtin_inff());
       }
       float4* o = (float4*)(y + (size_t)m * N + n0);
@@ -1809,10 +1817,10 @@ __device__ __forceinline__ void lmhead_rows_body(const _Float16* __restrict__ fr
 
 #define DEF_LMHEAD_ROWS(NAME, Q6, MT)                                                                          \
   extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void NAME(              \
-      const _Float16* __restrict__ frag, const float* __restrict__ rscale, const uint8_t* __restrict__ nib,    \
+      const _Float16* __restrict__ frag, const int32_t* __restrict__ rexp, const uint8_t* __restrict__ nib,    \
       const uint8_t* __restrict__ dsc, float* __restrict__ y, uint32_t M, uint32_t K, uint32_t N,              \
       const float* __restrict__ x, const float* __restrict__ gamma, float eps) {                               \
-    lmhead_rows_body<Q6, MT>(frag, rscale, nib, dsc, y, M, K, N, x, gamma, eps);                               \
+    lmhead_rows_body<Q6, MT>(frag, rexp, nib, dsc, y, M, K, N, x, gamma, eps);                                 \
   }
 DEF_LMHEAD_ROWS(smith_lmhead_q4_0_rows_m1, false, 1)
 DEF_LMHEAD_ROWS(smith_lmhead_q4_0_rows_m2, false, 2)

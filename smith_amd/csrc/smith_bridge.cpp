@@ -2115,14 +2115,14 @@ static int lmhead_rows(Ctx* c, const char* kernel, const float* x, uint32_t M, c
                        const void* nib, const void* d, float* y, uint32_t K, uint32_t N) {
   const uint32_t MT = M <= 16 ? 1 : (M <= 32 ? 2 : 4), M16 = (M + 15) / 16 * 16, KP = (K + 31) / 32;
   const size_t frag_bytes = (size_t)M16 * KP * 32 * 2 * 2;
-  if (ensure(c, &c->prep, &c->prep_bytes, frag_bytes + M16 * sizeof(float))) return -1;
+  if (ensure(c, &c->prep, &c->prep_bytes, frag_bytes + M16 * sizeof(int32_t))) return -1;
   void* frag = c->prep;
-  void* rs = (char*)c->prep + frag_bytes;
-  void* pargs[] = {&x, &norm_gamma, &eps, &frag, &rs, &M, &K};
+  void* re = (char*)c->prep + frag_bytes;
+  void* pargs[] = {&x, &norm_gamma, &eps, &frag, &re, &M, &K};
   if (launch(c, "smith_lmhead_split_rows", dim3(M16), dim3(256), pargs)) return -1;
   char name[64];
   snprintf(name, sizeof name, "%s_m%u", kernel, MT);
-  void* args[] = {&frag, &rs, &nib, &d, &y, &M, &K, &N, &x, &norm_gamma, &eps};
+  void* args[] = {&frag, &re, &nib, &d, &y, &M, &K, &N, &x, &norm_gamma, &eps};
   return launch(c, name, dim3((M + 16 * MT - 1) / (16 * MT), (N + 255) / 256), dim3(512), args);
 }
 

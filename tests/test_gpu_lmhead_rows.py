@@ -25,9 +25,10 @@ def _buf(a):
 
 
 class Head:
-    def __init__(self, kind, K, N, seed, scale=0.02):
+    def __init__(self, kind, K, N, seed, scale=0.02, w=None):
         L, ctx = device.lib, device.ops_ctx()
-        w = prng.randn((K, N), seed, std=scale)
+        if w is None:
+            w = prng.randn((K, N), seed, std=scale)
         t = O.GGML_Q4_0 if kind == "q4_0" else O.GGML_Q6_K
         blocks = O.quantize_rows(t, w)  # blocks run along vocab
         self.w = O.dequantize_tensor(t, blocks, K * N).reshape(K, N).astype(np.float64)
@@ -100,6 +101,36 @@ def test_rows_scales(kind, scale):
     y, ref = h.run(x, None), h.ref(x, None)
     for m in range(6):
         assert rel2(y[m], ref[m]) <= BAR, m
+    h.close()
+
+
+@pytest.mark.parametrize("kind", ["q4_0", "q6_k"])
+def test_rows_of_any_size(kind):
+    """Rows from next to the smallest f32 numbers to next to the largest."""
+    K, N = 1024, 512
+    h = Head(kind, K, N, 828)
+    x = prng.randn((6, K), 829) * np.float32([[1e-36], [1e-33], [1e-32], [1e-30], [1e33], [3e35]])
+    y, ref = h.run(x, None), h.ref(x, None)
+    for m in range(6):
+        assert rel2(y[m].astype(np.float64), ref[m]) <= BAR, m
+    h.close()
+
+
+@pytest.mark.parametrize("kind", ["q4_0", "q6_k"])
+def test_rows_outlier_at_zero_weights(kind):
+    """An element far above its row that meets zero weights: the outputs of
+    those columns come from the other elements alone, which keep their bits."""
+    K, N, at = 1024, 1024, 5
+    w = prng.randn((K, N), 830, std=0.02)
+    w[at, :N // 2] = 0.0
+    h = Head(kind, K, N, 0, w=w)
+    assert not h.w[at, :N // 2].any()
+    x = prng.randn((4, K), 831)
+    x[:, at] = [1e2, 1e4, 1e6, 1e8]
+    y, ref = h.run(x, None), h.ref(x, None)
+    for m in range(4):
+        assert rel2(y[m, :N // 2], ref[m, :N // 2]) <= BAR, m
+        assert rel2(y[m, N // 2:], ref[m, N // 2:]) <= BAR, m
     h.close()
 
 
