@@ -1512,8 +1512,9 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 //     (c, kq) of an MFMA takes output octet c and row octet kq, and fragment f
 //     of the eight it forms is output 8c + f: a lane ends with eight
 //     consecutive outputs of a row.
-// An output that is not finite (a weight beyond the f16 range, an infinite or
-// NaN x) is redone in f32 as the single-row heads compute it.
+// A row with an output that is not finite (a weight beyond the f16 range, an
+// infinite or NaN x) is redone in f32 as the single-row heads compute it, by
+// the whole workgroup over its 256 columns (lmhead_row_f32).
 // Bounded by the MFMAs: per 32 rows k, 32 MT of them (512 MT clocks) beside
 // ~170 (Q4_0) / ~430 (Q6_K) vector instructions.  K = 3072, N = 32000, 128
 // rows: Q4_0 103 us, Q6_K 113 us, where row by row took 128 launches of 18 /
@@ -1590,46 +1591,86 @@ extern "C" __global__ __launch_bounds__(256) void smith_lmhead_split_rows(const 
   }
 }
 
-// the f32 value of output n of row xr (after the norm), as the single-row
-// heads form it
-template <bool Q6>
-__device__ __forceinline__ float lmh_f32(const float* __restrict__ xr, const float* __restrict__ gamma, float eps,
-                         const uint8_t* __restrict__ nib, const uint8_t* __restrict__ dsc, uint32_t K, uint32_t N,
-                         uint32_t n) {
-  float rms = 1.f, ss = 0.f;
-  if (gamma) {
-    for (uint32_t k = 0; k < K; k++) ss = __builtin_fmaf(xr[k], xr[k], ss);
-    rms = 1.0f / __builtin_sqrtf(ss / (float)K + eps);
-  }
-  size_t ohb = 0, osc = 0, od = 0, tot;
-  if (Q6) lmh6_offsets(K, N, &ohb, &osc, &od, &tot);
-  const uint32_t vb = n / 32, sub = n % 32 / 8, e = n % 8;
-  float acc = 0.f, corr = 0.f;
-  for (uint32_t k = 0; k < K; k++) {
-    const float xv = gamma ? xr[k] * rms * gamma[k] : xr[k];
-    const size_t g = ((size_t)(k / 8) * (N / 32) + vb) * 4 + sub;
-    const uint32_t w = *(const uint32_t*)(nib + g * 32 + (k % 8) * 4);
-    uint32_t q = (w >> (4 * e)) & 15u;
-    float c;
-    if (Q6) {
-      q |= ((*(const uint16_t*)(nib + ohb + g * 16 + (k % 8) * 2) >> (2 * e)) & 3u) << 4;
-      const float d = (float)((const _Float16*)(nib + od))[(size_t)(n / 256) * K + k];
-      c = xv * (d * (float)((const int8_t*)(nib + osc))[(size_t)(n / 16) * K + k]);
-    } else {
-      c = xv * (float)((const _Float16*)dsc)[((size_t)(k / 8) * (N / 32) + vb) * 8 + k % 8];
-    }
-    corr += c;
-    acc = __builtin_fmaf(c, (float)q, acc);
-  }
-  return __builtin_fmaf(Q6 ? -32.0f : -8.0f, corr, acc);
-}
-
 // what a lane reads for eight rows k of its eight outputs
 template <bool Q6>
 struct LmhW {
   u32x4 n[2], h, d;
   uint2 sc;
 };
+
+// octet o of the rows, outputs nc .. nc + 7
+template <bool Q6>
+__device__ __forceinline__ LmhW<Q6> lmh_load(const uint8_t* __restrict__ nib, const uint8_t* __restrict__ dsc,
+                                             uint32_t K, uint32_t N, uint32_t nc, uint32_t o) {
+  LmhW<Q6> w;
+  const uint32_t NB = N / 32, vb = nc / 32, sub = nc % 32 / 8;
+  const size_t g = ((size_t)o * NB + vb) * 4 + sub;
+  w.n[0] = *(const u32x4*)(nib + g * 32);
+  w.n[1] = *(const u32x4*)(nib + g * 32 + 16);
+  if constexpr (Q6) {
+    size_t ohb, osc, od, tot;
+    lmh6_offsets(K, N, &ohb, &osc, &od, &tot);
+    w.h = *(const u32x4*)(nib + ohb + g * 16);
+    w.sc = *(const uint2*)(nib + osc + (size_t)(nc / 16) * K + 8 * o);
+    w.d = *(const u32x4*)(nib + od + ((size_t)(nc / 256) * K + 8 * o) * 2);
+  } else {
+    w.d = *(const u32x4*)(dsc + ((size_t)o * NB + vb) * 16);
+  }
+  return w;
+}
+
+// Outputs c0 .. c0 + 255 of one row in f32, the single-row heads' arithmetic:
+// the workgroup's 512 threads as 32 output octets x 16 shares of the rows k.
+// lds: 16 x 256 floats.
+template <bool Q6>
+__device__ __forceinline__ void lmhead_row_f32(const float* __restrict__ xr, const float* __restrict__ gamma,
+                                               float eps, const uint8_t* __restrict__ nib,
+                                               const uint8_t* __restrict__ dsc, float* __restrict__ yr, uint32_t K,
+                                               uint32_t N, uint32_t c0, float* lds) {
+  const uint32_t tid = threadIdx.x, share = tid / 32, n0 = c0 + tid % 32 * 8, nc = n0 < N ? n0 : N - 8;
+  float rms = 1.f;
+  if (gamma) {
+    float ss = 0.f;
+    for (uint32_t k = tid; k < K; k += 512) ss = __builtin_fmaf(xr[k], xr[k], ss);
+    ss = sum64_lanes(ss);
+    if (tid % 64 == 0) lds[tid / 64] = ss;
+    __syncthreads();
+    float tot = 0.f;
+    for (int w = 0; w < 8; w++) tot += lds[w];
+    rms = 1.0f / __builtin_sqrtf(tot / (float)K + eps);
+    __syncthreads();
+  }
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, corr = 0.f;
+#pragma unroll 2
+  for (uint32_t o = share; o < K / 8; o += 16) {
+    const LmhW<Q6> w = lmh_load<Q6>(nib, dsc, K, N, nc, o);
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+      const uint32_t k = 8 * o + r;
+      const float xv = gamma ? xr[k] * rms * gamma[k] : xr[k];
+      float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.d[r / 2] >> (16 * (r & 1))));
+      if constexpr (Q6) d *= (float)(int8_t)((r < 4 ? w.sc.x : w.sc.y) >> (8 * (r & 3)));
+      const float c = xv * d;
+      corr += c;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        uint32_t q = (w.n[r / 4][r % 4] >> (4 * e)) & 15u;
+        if constexpr (Q6) q |= ((w.h[r / 2] >> (16 * (r & 1) + 2 * e)) & 3u) << 4;
+        acc[e] = __builtin_fmaf(c, (float)q, acc[e]);
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; e++) lds[share * 256 + tid % 32 * 8 + e] = __builtin_fmaf(Q6 ? -32.0f : -8.0f, corr, acc[e]);
+  __syncthreads();
+  if (tid < 256 && c0 + tid < N) {
+    float v = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) v += lds[i * 256 + tid];
+    yr[c0 + tid] = v;
+  }
+  __syncthreads();
+}
 
 template <bool Q6, int MT>
 __device__ __forceinline__ void lmhead_rows_body(const _Float16* __restrict__ frag, const int32_t* __restrict__ rexp,
@@ -1639,33 +1680,20 @@ __device__ __forceinline__ void lmhead_rows_body(const _Float16* __restrict__ fr
                                                 float eps) {
   typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
   __shared__ f32x4_t red[4 * MT * 8 * 64];
+  __shared__ uint32_t bad[2];  // rows of this workgroup with an output that is not finite
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t wn = wave & 1, wk = wave >> 1;
   const uint32_t c = lane & 15, kq = lane >> 4;
-  const uint32_t NB = N / 32, KO = K / 8, KP = (K + 31) / 32;
+  const uint32_t KO = K / 8, KP = (K + 31) / 32;
   const uint32_t m0 = blockIdx.x * 16 * MT, n0 = blockIdx.y * 256 + wn * 128 + 8 * c;
   const uint32_t nc = n0 < N ? n0 : N - 8;  // lanes past N read the last outputs and store nothing
-  const uint32_t vb = nc / 32, sub = nc % 32 / 8;
   const uint32_t per = (KP + 3) / 4, s0 = wk * per < KP ? wk * per : KP, s1 = s0 + per < KP ? s0 + per : KP;
   const size_t plane = (size_t)((M + 15) / 16) * KP * 512;
-  size_t ohb = 0, osc = 0, od = 0, tot;
-  if (Q6) lmh6_offsets(K, N, &ohb, &osc, &od, &tot);
+  if (tid < 2) bad[tid] = 0;
 
-  auto loadw = [&](uint32_t s) {
-    LmhW<Q6> w;
-    const uint32_t o = 4 * s + kq < KO ? 4 * s + kq : KO - 1;  // x is zero past K
-    const size_t g = ((size_t)o * NB + vb) * 4 + sub;
-    w.n[0] = *(const u32x4*)(nib + g * 32);
-    w.n[1] = *(const u32x4*)(nib + g * 32 + 16);
-    if constexpr (Q6) {
-      w.h = *(const u32x4*)(nib + ohb + g * 16);
-      w.sc = *(const uint2*)(nib + osc + (size_t)(nc / 16) * K + 8 * o);
-      w.d = *(const u32x4*)(nib + od + ((size_t)(nc / 256) * K + 8 * o) * 2);
-    } else {
-      w.d = *(const u32x4*)(dsc + ((size_t)o * NB + vb) * 16);
-    }
-    return w;
+  auto loadw = [&](uint32_t s) {  // x is zero past K
+    return lmh_load<Q6>(nib, dsc, K, N, nc, 4 * s + kq < KO ? 4 * s + kq : KO - 1);
   };
   auto loada = [&](u32x4 (&a)[MT][2], uint32_t s) {
 #pragma unroll
@@ -1787,31 +1815,34 @@ __device__ __forceinline__ void lmhead_rows_body(const _Float16* __restrict__ fr
     }
     __syncthreads();
   }
-  if (wk != 0 || n0 >= N) return;
-  bool bad = false;
+  if (wk == 0 && n0 < N) {
 #pragma unroll
-  for (int mt = 0; mt < MT; mt++)
+    for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const uint32_t m = m0 + 16 * mt + 4 * kq + e;
-      if (m >= M) continue;
-      const int re = rexp[m];
-      float v[8];
+      for (int e = 0; e < 4; e++) {
+        const uint32_t i = 16 * mt + 4 * kq + e, m = m0 + i;
+        if (m >= M) continue;
+        const int re = rexp[m];
+        float v[8];
+        bool finite = true;
 #pragma unroll
-      for (int f = 0; f < 8; f++) {
-        v[f] = __builtin_ldexpf(acc[mt][f][e], re);
-        bad |= !(__builtin_fabsf(v[f]) < __builtin_inff());
+        for (int f = 0; f < 8; f++) {
+          v[f] = __builtin_ldexpf(acc[mt][f][e], re);
+          finite &= __builtin_fabsf(v[f]) < __builtin_inff();
+        }
+        float4* o = (float4*)(y + (size_t)m * N + n0);
+        o[0] = make_float4(v[0], v[1], v[2], v[3]);
+        o[1] = make_float4(v[4], v[5], v[6], v[7]);
+        if (!finite) atomicOr(&bad[i / 32], 1u << (i % 32));
       }
-      float4* o = (float4*)(y + (size_t)m * N + n0);
-      o[0] = make_float4(v[0], v[1], v[2], v[3]);
-      o[1] = make_float4(v[4], v[5], v[6], v[7]);
-    }
-  if (!bad) return;
-#pragma unroll 1
-  for (uint32_t i = 0; i < 32 * MT; i++) {  // this lane's own outputs again
-    const uint32_t m = m0 + 16 * (i / 32) + 4 * kq + i / 8 % 4, n = n0 + i % 8;
-    if (m < M && !(__builtin_fabsf(y[(size_t)m * N + n]) < __builtin_inff()))
-      y[(size_t)m * N + n] = lmh_f32<Q6>(x + (size_t)m * K, gamma, eps, nib, dsc, K, N, n);
+  }
+  __syncthreads();
+  // the same rows in every thread
+  uint64_t rest = (uint64_t)__builtin_amdgcn_readfirstlane(bad[1]) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane(bad[0]);
+  while (rest) {
+    const uint32_t m = m0 + (uint32_t)__builtin_ctzll(rest);
+    rest &= rest - 1;
+    lmhead_row_f32<Q6>(x + (size_t)m * K, gamma, eps, nib, dsc, y + (size_t)m * N, K, N, blockIdx.y * 256, (float*)red);
   }
 }
 

@@ -151,3 +151,38 @@ def test_rows_not_finite(kind):
                 f = ~np.isnan(want[m])
                 assert np.array_equal(y[m][f], want[m][f]), m
     h.close()
+
+
+@pytest.mark.parametrize("kind", ["q4_0", "q6_k"])
+@pytest.mark.parametrize("M", [17, 64])
+def test_rows_not_finite_time(kind, M):
+    """Rows that are redone in f32 cost no more than the same rows through the
+    single-row head (twice that: room for the clocks)."""
+    K, N = 2048, 16384
+    h = Head(kind, K, N, 832)
+    x = prng.randn((M, K), 833)
+    x[:, 9] = np.nan
+    us = []
+    for rows, name in ((True, "smith_lmhead_%s_rows_m" % kind), (False, "smith_lmhead_%s_nb" % kind)):
+        assert np.isnan(h.run(x, None, rows)).all()
+        device.profile_kernels(True)
+        h.run(x, None, rows)
+        ms, _ = device.profile_read(name)
+        device.profile_read("")
+        device.profile_kernels(False)
+        us.append(ms)
+    assert us[0] <= 2 * us[1], us
+    h.close()
+
+
+@pytest.mark.parametrize("kind", ["q4_0", "q6_k"])
+def test_rows_weights_beyond_f16(kind):
+    """Weights above the f16 range: every row is redone in f32."""
+    K, N = 264 if kind == "q4_0" else 272, 768
+    h = Head(kind, K, N, 834, 6e4)
+    assert np.abs(h.w).max() > 65504
+    for M in (5, 33, 70):
+        x = prng.randn((M, K), 835)
+        g = 1 + prng.randn((K,), 836, std=0.1)
+        assert rel2(h.run(x, g), h.ref(x, g)) <= BAR, M
+    h.close()
