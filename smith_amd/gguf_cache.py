@@ -247,6 +247,8 @@ class _Engine:
         """Prompt rows in chunks of <= 256 (attention keeps a chunk's keys in
         LDS); returns the logits of every row if asked, else of the last."""
         n = len(tokens)
+        if all_logits and not n:
+            raise ValueError("prefill of an empty prompt: there are no logits to return")
         step, dim, vocab = _chunk_rows(self.cfg), self.cfg["dim"], self.cfg["vocabSize"]
         logits = np.empty((n, vocab), np.float32) if all_logits else None
         if all_logits and (self.row_logits is None or self.row_logits.shape[0] < min(n, step)):

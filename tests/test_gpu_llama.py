@@ -53,6 +53,12 @@ def test_prefill_and_decode_logits(q4):
         assert normwise_rel_err(g, w) <= TOL, i
 
 
+def test_empty_prompt_is_refused(q4):
+    m = loadGGUF(q4)
+    with pytest.raises(ValueError):
+        m.forwardPrefill([], m.createCache())
+
+
 def test_repeated_prefill_is_deterministic(q4):
     """The same prompt into the same caches three times: the logits agree
     bit for bit (fixed split-K and reduction orders), and with the oracle."""
