@@ -37,6 +37,10 @@ FUSED_GREEDY = os.environ.get("SMITH_FUSED_GREEDY", "1") != "0"
 PREP_NEXT = os.environ.get("SMITH_PREP_NEXT", "1") != "0"
 
 PREFILL_CHUNK = 256
+# Device memory an engine keeps for the logits of a prompt's rows: a whole
+# chunk's up to a vocabulary of 32768, fewer rows (at least 64, one LM head
+# tile) above it.
+ROW_LOGITS_BYTES = 32 << 20
 
 
 def _chunk_rows(cfg):
@@ -74,7 +78,7 @@ class _Engine:
         self.attn = DeviceArray((R, dim))
         self.h = DeviceArray((R, ffn))
         self.logits = DeviceArray((cfg["vocabSize"],))
-        self.row_logits = None  # [rows, vocab] of a prompt's logits, made for the first such call
+        self.row_logits = None  # [block, vocab] of a prompt's logits, made for the first such call
         self.pos = DeviceArray((1,), np.int32)
         self.count = DeviceArray((1,), np.int32)
         self.tokens = DeviceArray((cfg["maxSeqLen"] + 1,), np.int32)
@@ -226,22 +230,23 @@ class _Engine:
         device.check(device.lib.smith_embed(device.ops_ctx(), model["embedding"].ptr, self.tok_in.ptr, self.x.ptr,
                                             len(t), self.cfg["dim"], a0, g0), "embed")
 
-    def lm_head_rows(self, model, M, out_ptr):
-        """lm_head of rows x[0:M] into [M, vocab] at out_ptr: one launch over
+    def lm_head_rows(self, model, r0, M, out_ptr):
+        """lm_head of rows x[r0:r0+M] into [M, vocab] at out_ptr: one launch over
         the rows for a Q4_0 or Q6_K head, else row by row."""
         cfg, ctx = self.cfg, device.ops_ctx()
         head, g, eps = model["lmHead"], model["lnFGamma"].ptr, model["normEps"]
+        x = self.x.ptr + r0 * cfg["dim"] * 4
         if head["kind"] == "q4_0_nb":
-            rc = device.lib.smith_lmhead_q4_0_rows(ctx, self.x.ptr, M, g, eps, head["nib"].ptr, head["d"].ptr, out_ptr,
+            rc = device.lib.smith_lmhead_q4_0_rows(ctx, x, M, g, eps, head["nib"].ptr, head["d"].ptr, out_ptr,
                                                    cfg["dim"], cfg["vocabSize"])
             device.check(rc, "lm head")
         elif head["kind"] == "q6_k_nb":
-            rc = device.lib.smith_lmhead_q6_k_rows(ctx, self.x.ptr, M, g, eps, head["planes"].ptr, out_ptr, cfg["dim"],
+            rc = device.lib.smith_lmhead_q6_k_rows(ctx, x, M, g, eps, head["planes"].ptr, out_ptr, cfg["dim"],
                                                    cfg["vocabSize"])
             device.check(rc, "lm head")
         else:
             for r in range(M):
-                self.lm_head(model, self.x.ptr + r * cfg["dim"] * 4, out_ptr + r * cfg["vocabSize"] * 4)
+                self.lm_head(model, x + r * cfg["dim"] * 4, out_ptr + r * cfg["vocabSize"] * 4)
 
     def prefill(self, model, tokens, caches, all_logits=False):
         """Prompt rows in chunks of <= 256 (attention keeps a chunk's keys in
@@ -251,20 +256,21 @@ class _Engine:
             raise ValueError("prefill of an empty prompt: there are no logits to return")
         step, dim, vocab = _chunk_rows(self.cfg), self.cfg["dim"], self.cfg["vocabSize"]
         logits = np.empty((n, vocab), np.float32) if all_logits else None
-        if all_logits and (self.row_logits is None or self.row_logits.shape[0] < min(n, step)):
-            from .gguf_loader import DeviceArray
-            old, self.row_logits = self.row_logits, None
-            if old is not None:
-                device.release_buffer(old.ptr)
-            self.row_logits = DeviceArray((min(n, step), vocab))
+        if all_logits:
+            if self.row_logits is None:
+                from .gguf_loader import DeviceArray
+                self.row_logits = DeviceArray((min(step, max(64, ROW_LOGITS_BYTES // (vocab * 4) // 64 * 64)), vocab))
+            block = self.row_logits.shape[0]
         for r0 in range(0, n, step):
             r1 = min(n, r0 + step)
             self.embed(model, tokens[r0:r1])
             self.set_pos(r0)
             self.layers(model, caches, r1 - r0)
             if all_logits:
-                self.lm_head_rows(model, r1 - r0, self.row_logits.ptr)
-                device.download_into(logits[r0:r1], self.row_logits.ptr)
+                for b0 in range(r0, r1, block):
+                    b1 = min(r1, b0 + block)
+                    self.lm_head_rows(model, b0 - r0, b1 - b0, self.row_logits.ptr)
+                    device.download_into(logits[b0:b1], self.row_logits.ptr)
         last = (n - 1) % step
         if not all_logits:
             self.lm_head(model, self.x.ptr + last * dim * 4)

@@ -10,6 +10,7 @@ import pytest
 
 from oracle import llama_oracle as LO
 from oracle.oracle import normwise_rel_err
+from smith_amd import gguf_cache
 from smith_amd.gguf_loader import loadGGUF
 from tests.llama_fixtures import write_tiny_llama
 
@@ -57,6 +58,24 @@ def test_empty_prompt_is_refused(q4):
     m = loadGGUF(q4)
     with pytest.raises(ValueError):
         m.forwardPrefill([], m.createCache())
+
+
+def test_row_logits_buffer(q4, monkeypatch):
+    """One buffer of bounded size for every prompt length; prompts of more
+    rows than it holds go through it in blocks, with the same logits."""
+    prompt = [(7 * i + 3) % SMALL["vocab"] for i in range(150)]
+    m = loadGGUF(q4)
+    e = gguf_cache._engine(m.model)
+    m.forwardPrefill(prompt[:2], m.createCache())
+    ptr = e.row_logits.ptr
+    assert e.row_logits.nbytes <= max(gguf_cache.ROW_LOGITS_BYTES, 64 * SMALL["vocab"] * 4)
+    whole = m.forwardPrefill(prompt, m.createCache())["logits"]
+    assert e.row_logits.ptr == ptr
+    monkeypatch.setattr(gguf_cache, "ROW_LOGITS_BYTES", 1)
+    m2 = loadGGUF(q4)
+    blocks = m2.forwardPrefill(prompt, m2.createCache())["logits"]
+    assert gguf_cache._engine(m2.model).row_logits.shape[0] == 64
+    assert np.array_equal(blocks, whole)
 
 
 def test_repeated_prefill_is_deterministic(q4):
