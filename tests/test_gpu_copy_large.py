@@ -1,6 +1,7 @@
 """smith_copy_d2h through the pinned slots (4 MB and up): every byte, at the
 edges of the threshold, the 1 MB chunks and the eight slots, from an offset,
-in order with work enqueued before it, and from two threads at once; into pinned memory, directly."""
+in order with work enqueued before it, and from two threads at once; into pinned memory, directly;
+and behind a long queue of earlier work."""
 import ctypes
 import threading
 import time
@@ -80,3 +81,27 @@ def test_pinned_destination():
     assert np.array_equal(out[1000:], a[1000:]) and not out[:1000].any()
     device.release_buffer(b)
     hip.hipHostFree(dst)
+
+
+def test_waits_in_one_thread():
+    """While the stream still works on what was enqueued before the copy, one
+    thread waits (the helpers would make it four)."""
+    M, N, K = 2048, 4096, 4096
+    a, out, b = device.alloc(M * K * 4), device.alloc(M * N * 4), device.alloc(8 * MB)
+    w = device.alloc(K // 32 * N * 24)
+    for buf, n in ((a, M * K * 4), (w, K // 32 * N * 24), (b, 8 * MB)):
+        device.check(device.lib.smith_fill_zero(device.ops_ctx(), buf, n))
+    device.download(b, 8 * MB, np.uint32)
+    for _ in range(2):  # the first round makes the scratch
+        device.sync()
+        wall, cpu = time.perf_counter(), time.process_time()
+        for _ in range(400):
+            device.check(device.lib.smith_matmul_q4(device.ops_ctx(), a, w, out, M, N, K, K // 32))
+        queued = time.perf_counter() - wall
+        device.download(b, 8 * MB, np.uint32)
+        wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    print("waits", queued, wall, cpu)
+    assert wall > 2 * queued  # the copy did wait for the GPU
+    assert cpu <= 1.6 * wall, (cpu, wall)
+    for buf in (a, out, b, w):
+        device.release_buffer(buf)
