@@ -164,12 +164,21 @@ hipEvent_t pooled_event(Ctx* c) {
   return e;
 }
 
+// Around runtime calls whose failure is an answer: takes the error that they
+// leave with the thread out again, unless one was there before (another
+// user's, who still has to find an error).
+struct QuietErrors {
+  const bool clean = hipPeekAtLastError() == hipSuccess;
+  ~QuietErrors() {
+    if (clean) (void)hipGetLastError();
+  }
+};
+
 // Op kernels may live in any loaded code object (smith_kernels.hsaco,
 // smith_llama.hsaco, ...): first match in load order wins.  Found once per
 // name and kept by the context: a lookup that misses in an earlier code object
-// is slow and leaves hipErrorNotFound behind (taken out here, so that another
-// user of the runtime in this thread does not see it), and the kernels of the
-// later objects would pay for it on every launch.
+// is slow and leaves hipErrorNotFound behind (QuietErrors), and the kernels of
+// the later objects would pay for it on every launch.
 int find_kernel(Ctx* c, const char* name, hipFunction_t* out) {
   const auto known = c->kernels.find(name);
   if (known != c->kernels.end()) {
@@ -177,6 +186,7 @@ int find_kernel(Ctx* c, const char* name, hipFunction_t* out) {
     return 0;
   }
   if (c->libs.empty()) return fail(c, "smith: no code object loaded (call smith_load_library first)");
+  QuietErrors quiet;
   for (Library* lib : c->libs) {
     hipFunction_t f;
     if (hipModuleGetFunction(&f, lib->mod, name) == hipSuccess) {
@@ -184,7 +194,6 @@ int find_kernel(Ctx* c, const char* name, hipFunction_t* out) {
       *out = f;
       return 0;
     }
-    (void)hipGetLastError();
   }
   return fail(c, "smith: kernel '%s' not found in any loaded code object", name);
 }
@@ -816,18 +825,15 @@ constexpr int STAGE_SLOTS = 8, STAGE_HELPERS = 3;
 static bool stage_ready(Ctx* c) {
   std::lock_guard<std::mutex> lk(c->stage_mu);
   if (c->stage) return true;
+  QuietErrors quiet;
   static_assert(sizeof c->stage_ev / sizeof c->stage_ev[0] == STAGE_SLOTS, "an event per slot");
   for (hipEvent_t& ev : c->stage_ev)
     if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
-      (void)hipGetLastError();
       ev = nullptr;
       return false;
     }
   void* p = nullptr;
-  if (hipHostMalloc(&p, STAGE_SLOTS * STAGE_CHUNK, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
+  if (hipHostMalloc(&p, STAGE_SLOTS * STAGE_CHUNK, hipHostMallocDefault) != hipSuccess) return false;
   c->stage = (uint8_t*)p;
   return true;
 }
@@ -835,10 +841,9 @@ static bool stage_ready(Ctx* c) {
 // ordinary host memory: not pinned, managed or on a device, where the runtime
 // copies directly (64 MB into pinned memory 1.19 ms, through the slots 2.20)
 static bool pageable(const void* p) {
+  QuietErrors quiet;
   hipPointerAttribute_t at{};
-  if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type == hipMemoryTypeUnregistered;
-  (void)hipGetLastError();
-  return true;
+  return hipPointerGetAttributes(&at, p) != hipSuccess || at.type == hipMemoryTypeUnregistered;
 }
 
 static int large_d2h(Ctx* c, uint8_t* dst, const uint8_t* src, uint64_t bytes) {

@@ -215,3 +215,29 @@ def test_first_split_k_calls_on_a_fresh_context():
             device.release_buffer(b)
     finally:
         lib.smith_destroy(c)
+
+
+def test_kernel_lookup_leaves_the_last_error():
+    """Looking a kernel up past the code objects that lack it leaves no HIP
+    error behind, and one that another user of the runtime still has to read
+    stays an error."""
+    hip, lib = ctypes.CDLL("libamdhip64.so.7"), device.lib
+    M, N, K = 64, 64, 64
+    a, w, o = device.alloc(M * K * 4), device.alloc(K // 32 * N * 24), device.alloc(M * N * 4)
+    for b, n in ((a, M * K * 4), (w, K // 32 * N * 24)):
+        device.check(lib.smith_fill_zero(device.ops_ctx(), b, n))
+    device.sync()
+    for pending in (False, True):
+        c = lib.smith_init()
+        for path in (device.CODE_OBJECT_PATH, device.LLAMA_CODE_OBJECT_PATH, device.GEMM_CODE_OBJECT_PATH):
+            assert lib.smith_load_library(c, path.encode())
+        hip.hipGetLastError()
+        if pending:
+            assert hip.hipSetDevice(9999) != 0
+            assert hip.hipPeekAtLastError() != 0
+        assert lib.smith_matmul_q4(c, a, w, o, M, N, K, K // 32) == 0, lib.smith_last_error(c)
+        assert lib.smith_sync(c) == 0
+        assert (hip.hipGetLastError() != 0) == pending
+        lib.smith_destroy(c)
+    for b in (a, w, o):
+        device.release_buffer(b)
