@@ -568,7 +568,11 @@ constexpr size_t NOALLOC_PREP_BYTES = 4u << 20;
 // it also prepares the next GEMM's rows, a launch less there, and 0.5 us).
 // (Measured on either side: Q4S M = 512, 14336 x 4096 TM = 8 without splits
 // 71 us, 16 with two 81; Q8 M = 301 10 with two 61, 8 without 69; Q4S M =
-// 2048, 4096 x 14336 both 252.)
+// 2048, 4096 x 14336 both 252.)  Partials take at most 64 MiB, which the
+// context keeps: what 256 workgroups of 256 x 256 tiles take; under 1 % of the
+// shapes up to M = 2048, N = K = 14336 would split further, for 4 % on average.
+constexpr size_t GEMM3_WS_BYTES = 64u << 20;
+
 uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, bool fused, uint32_t* ks_out) {
   const double conv = fmt == FQ8 || fmt > FQ40T ? 0.45 : 0.35;
   static const uint32_t tms[] = {2, 4, 6, 8, 10, 12, 14, 16};
@@ -581,6 +585,7 @@ uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, bool fused, uin
     for (uint32_t ks = 1; ks <= 16 && (ks == 1 || S / ks >= 4); ks++) {
       const uint32_t sps = (S + ks - 1) / ks;
       if ((S + sps - 1) / sps != ks) continue;  // the same stages per split as a smaller count
+      if (ks > 1 && (size_t)ks * M * N * sizeof(float) > GEMM3_WS_BYTES) break;
       // the static scratch takes every plan of the shapes whose activations
       // it holds, so that both matmulQ4 entry points run the same one
       if (ks > 1 && fmt == FQ4S && (size_t)M * S * 128 <= NOALLOC_PREP_BYTES &&
@@ -637,47 +642,44 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
     if (!(pre && perm) && launch(c, perm ? "smith_gemm_prep_a_perm" : "smith_gemm_prep_a", dim3(M), dim3(256), args))
       return -1;
   }
-  // tile choice: the biggest tile that still gives about one tile per CU
-  // (bigger tiles carry more MFMA work per K stage to cover load latency);
-  // small grids split K across workgroups (partials reduced after)
   auto ntiles = [&](uint32_t bm, uint32_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  uint32_t bm = 128, bn = 64;
-  if (ntiles(256, 256) >= 256) bm = 256, bn = 256;
-  else if (ntiles(256, 128) >= 200) bm = 256, bn = 128;
-  else if (ntiles(128, 128) >= 256) bm = 128, bn = 128;
-  if (g2 && M <= 128) bn = ntiles(128, 128) >= 128 ? 128 : 64;
-  if (g2 && bm == 256 && bn == 256) bn = 128;  // 256x256 spills registers on the high-bit formats
-  // M >= 256 on the register-staged kernel: 256x256 tiles (one 1024-thread
-  // workgroup per CU) and enough K splits to fill one wave of workgroups,
-  // each split at least 8 stages
-  const bool big = !g2 && M >= 256;
-  if (big) bm = bn = 256;
-  uint32_t tiles = ntiles(bm, bn);
   const uint32_t S = (K + 63) / 64;
-  uint32_t ks = 1;
-  if (big) {
-    ks = std::max<uint32_t>(1, std::min<uint32_t>(256 / tiles, S / 8));
-  } else if (g2 && bm == 128 && tiles < 512) {
-    // about 450 workgroups, at least 6 stages per split (measured at M = 128)
-    ks = std::min<uint32_t>(std::max<uint32_t>(1, (448 + tiles / 2) / tiles), std::max<uint32_t>(1, S / 6));
-  } else if (bm == 128 && bn == 64 && tiles < 512) {
-    ks = std::min<uint32_t>((512 + tiles - 1) / tiles, std::max<uint32_t>(1, S / 8));
-  }
-  uint32_t sps = (S + ks - 1) / ks;
-  ks = (S + sps - 1) / sps;
-  if (ks > 1 && ensure(c, (void**)&c->ws, &c->ws_bytes, (size_t)ks * M * N * sizeof(float))) return -1;
+  uint32_t tiles, threads, ks = 1;
   char name[64];
-  snprintf(name, sizeof name, "smith_gemm%s_%s_m%u_n%u", g2 ? "2" : "", fmt_tag(fmt), bm, bn);
-  uint32_t threads = 64 * (bm / 64) * (bn / (bn >= 128 ? 64 : 32));
-  // Which shapes the static scratch takes is still decided by the tiles and
-  // splits above.
   if (g3) {
     const uint32_t tm = gemm3_plan(fmt, M, N, S, want_next && ep.mode != 0, &ks);
-    sps = (S + ks - 1) / ks;
-    if (ks > 1 && ensure(c, (void**)&c->ws, &c->ws_bytes, (size_t)ks * M * N * sizeof(float))) return -1;
     snprintf(name, sizeof name, "smith_gemm3_%s_m%u", fmt_tag(fmt), tm);
     tiles = ntiles(16 * tm, 256), threads = 512;
+  } else {
+    // tile choice: the biggest tile that still gives about one tile per CU
+    // (bigger tiles carry more MFMA work per K stage to cover load latency);
+    // small grids split K across workgroups (partials reduced after)
+    uint32_t bm = 128, bn = 64;
+    if (ntiles(256, 256) >= 256) bm = 256, bn = 256;
+    else if (ntiles(256, 128) >= 200) bm = 256, bn = 128;
+    else if (ntiles(128, 128) >= 256) bm = 128, bn = 128;
+    if (g2 && M <= 128) bn = ntiles(128, 128) >= 128 ? 128 : 64;
+    if (g2 && bm == 256 && bn == 256) bn = 128;  // 256x256 spills registers on the high-bit formats
+    // M >= 256 on the register-staged kernel: 256x256 tiles (one 1024-thread
+    // workgroup per CU) and enough K splits to fill one wave of workgroups,
+    // each split at least 8 stages
+    const bool big = !g2 && M >= 256;
+    if (big) bm = bn = 256;
+    tiles = ntiles(bm, bn);
+    if (big) {
+      ks = std::max<uint32_t>(1, std::min<uint32_t>(256 / tiles, S / 8));
+    } else if (g2 && bm == 128 && tiles < 512) {
+      // about 450 workgroups, at least 6 stages per split (measured at M = 128)
+      ks = std::min<uint32_t>(std::max<uint32_t>(1, (448 + tiles / 2) / tiles), std::max<uint32_t>(1, S / 6));
+    } else if (bm == 128 && bn == 64 && tiles < 512) {
+      ks = std::min<uint32_t>((512 + tiles - 1) / tiles, std::max<uint32_t>(1, S / 8));
+    }
+    snprintf(name, sizeof name, "smith_gemm%s_%s_m%u_n%u", g2 ? "2" : "", fmt_tag(fmt), bm, bn);
+    threads = 64 * (bm / 64) * (bn / (bn >= 128 ? 64 : 32));
   }
+  const uint32_t sps = (S + ks - 1) / ks;
+  ks = (S + sps - 1) / sps;
+  if (ks > 1 && ensure(c, (void**)&c->ws, &c->ws_bytes, (size_t)ks * M * N * sizeof(float))) return -1;
   const void* pA = c->a16;
   const void* pB = B;
   const void* pD = D;

@@ -117,7 +117,9 @@ def test_noalloc_ignores_prepared_operand_hint():
 # (one-launch GEMV with K splits), M=16 / 32 (activation staging + partials),
 # M=64 (f16 staging of the GEMM); each pair: second call smaller
 CASES = [((1, 4096, 14336), (1, 1024, 4096)), ((8, 4096, 4096), (4, 1024, 2048)),
-         ((32, 4096, 4096), (16, 2048, 4096)), ((64, 1024, 4096), (64, 512, 1024))]
+         ((32, 4096, 4096), (16, 2048, 4096)), ((64, 1024, 4096), (64, 512, 1024)),
+         # f16 activations of 4 MiB and no K splits; K splits held to the region
+         ((512, 14336, 4096), (300, 1000, 4096))]
 
 
 @pytest.mark.parametrize("first,second", CASES)
@@ -158,4 +160,28 @@ def test_noalloc_rejects_oversized_scratch():
     assert "smith_matmul_q4_noalloc" in msg and "static scratch" in msg, msg
     device.sync()
     for b in (bq, ba, bo):
+        device.release_buffer(b)
+
+
+@pytest.mark.parametrize("M,N,K,splits", [(512, 14336, 4096, 0), (2047, 10145, 12352, 64 << 20), (64, 4096, 4096, 64 << 20)])
+@pytest.mark.parametrize("fmt", ["q4", "q8"])
+def test_gemm_scratch(fmt, M, N, K, splits):
+    """What a context keeps after a GEMM: the f16 activations and the split
+    partials of the plan that ran (none without splits, else at most 64 MiB),
+    each rounded up to 1 MiB."""
+    lib = device.lib
+    rec = 24 if fmt == "q4" else 34
+    c = _fresh_ctx()
+    bufs = []
+    for n in (M * K * 4, K // 32 * N * rec // 4 * 4, M * N * 4):
+        bufs.append(device.alloc(n + 64))
+        device.check(lib.smith_fill_zero(device.ops_ctx(), bufs[-1], n))
+    device.sync()
+    print("gemm scratch", fmt, M, N, K, flush=True)
+    fn = lib.smith_matmul_q4 if fmt == "q4" else lib.smith_matmul_q8
+    assert fn(c, *bufs, M, N, K, K // 32) == 0, lib.smith_last_error(c)
+    assert lib.smith_sync(c) == 0
+    assert lib.smith_allocated_size(c) <= M * K * 2 + splits + (2 << 20)
+    lib.smith_destroy(c)
+    for b in bufs:
         device.release_buffer(b)
