@@ -571,6 +571,9 @@ constexpr size_t NOALLOC_PREP_BYTES = 4u << 20;
 // 2048, 4096 x 14336 both 252.)  Partials take at most 64 MiB, which the
 // context keeps: what 256 workgroups of 256 x 256 tiles take; under 1 % of the
 // shapes up to M = 2048, N = K = 14336 would split further, for 4 % on average.
+// More than 16 splits where one tile or two would leave the chip idle (whole
+// calls, 64 rows: Q6_K 256 x 8192 16 splits 20.1 us, 32 17.8; Q8 64 x 14336 16
+// splits 20.2, 56 17.8).
 constexpr size_t GEMM3_WS_BYTES = 64u << 20;
 
 uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, bool fused, uint32_t* ks_out) {
@@ -581,8 +584,9 @@ uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, bool fused, uin
   *ks_out = 1;
   for (uint32_t tm : tms) {
     if (tm == 2 && M > 32) continue;  // a weight is converted once per row tile
+    if (tm > 2 && 16 * (tm - 2) >= M) break;  // the tile before holds every row
     const uint64_t tiles = (uint64_t)((M + 16 * tm - 1) / (16 * tm)) * ((N + 255) / 256);
-    for (uint32_t ks = 1; ks <= 16 && (ks == 1 || S / ks >= 4); ks++) {
+    for (uint32_t ks = 1; (ks <= 16 || (ks <= 64 && tiles * ks <= 256)) && (ks == 1 || S / ks >= 4); ks++) {
       const uint32_t sps = (S + ks - 1) / ks;
       if ((S + sps - 1) / sps != ks) continue;  // the same stages per split as a smaller count
       if (ks > 1 && (size_t)ks * M * N * sizeof(float) > GEMM3_WS_BYTES) break;

@@ -185,3 +185,22 @@ def test_gemm_scratch(fmt, M, N, K, splits):
     lib.smith_destroy(c)
     for b in bufs:
         device.release_buffer(b)
+
+
+@pytest.mark.parametrize("M,N,K,splits", [(64, 256, 14336, 56), (64, 256, 8192, 32)])
+def test_gemm_narrow_splits(M, N, K, splits):
+    """One tile over K in one split per four stages, not in 16: the partials
+    of that many splits."""
+    c = _fresh_ctx()
+    bufs = []
+    for n in (M * K * 4, K // 32 * N * 34, M * N * 4):
+        bufs.append(device.alloc(n))
+        device.check(device.lib.smith_fill_zero(device.ops_ctx(), bufs[-1], n))
+    device.sync()
+    assert device.lib.smith_matmul_q8(c, *bufs, M, N, K, K // 32) == 0, device.lib.smith_last_error(c)
+    assert device.lib.smith_sync(c) == 0
+    mib = 1 << 20
+    assert device.lib.smith_allocated_size(c) >= M * K * 2 + -(-splits * M * N * 4 // mib) * mib
+    device.lib.smith_destroy(c)
+    for b in bufs:
+        device.release_buffer(b)
