@@ -2157,6 +2157,22 @@ int smith_lmhead_q6_k_greedy(void* ctx, const float* x, const float* norm_gamma,
   return lmhead_q6_k(c, "smith_lmhead_q6_k_greedy", x, norm_gamma, eps, planes, logits, K, N, gt);
 }
 
+// A few rows of a head with few columns or a long K are faster one by one: a
+// workgroup of smith_lmhead_*_rows walks a quarter of K whatever N is, where
+// the single-row heads spread K over workgroups of their own.  us of a 16-row
+// tile (a pass of 256 workgroups: 65536 columns) against M single rows,
+// measured over K = 512 .. 8192, N = 256 .. 128256 and within 10 % of it where
+// the two are close (K = 3072, 2 rows by the tile / one by one: Q4_0 N = 2048
+// 38.8 / 18.0, 65536 42.3 / 60.0; Q6_K 56.7 / 25.8, 60.3 / 96.9).
+static bool rows_one_by_one(bool q6, uint32_t M, uint32_t K, uint32_t N) {
+  if (M > 16) return false;
+  const double kn = (double)K * N, passes = (N + 65535) / 65536;
+  const double tile = 8.5 + (q6 ? 0.0156 : 0.0095) * K * passes;
+  const double row = q6 ? std::max(11.9 + 1.7e-4 * K, 8.0 + 2.05e-7 * kn)
+                        : std::max(8.3 + 2.6e-4 * K, 4.6 + 6e-4 * K + 1.2e-7 * kn);
+  return M * row < tile;
+}
+
 // logits of M rows: the rows as split f16 operands, then the MFMA kernel.
 // 64 rows a workgroup from 33 rows up (an operand fetched once per 64 rows),
 // else the smallest tile that holds them.
@@ -2180,7 +2196,7 @@ int smith_lmhead_q4_0_rows(void* ctx, const float* x, uint32_t M, const float* n
   Ctx* c = (Ctx*)ctx;
   if (!c) return -1;
   const char* who = "smith_lmhead_q4_0_rows";
-  if (M <= 1 || ((uintptr_t)y & 15)) {
+  if (M <= 1 || ((uintptr_t)y & 15) || rows_one_by_one(false, M, K, N)) {
     for (uint32_t m = 0; m < M; m++)
       if (lmhead_q4_0(c, who, x + (size_t)m * K, norm_gamma, eps, nib, d, y + (size_t)m * N, K, N, GreedyTail{}))
         return -1;
@@ -2197,7 +2213,7 @@ int smith_lmhead_q6_k_rows(void* ctx, const float* x, uint32_t M, const float* n
   Ctx* c = (Ctx*)ctx;
   if (!c) return -1;
   const char* who = "smith_lmhead_q6_k_rows";
-  if (M <= 1 || ((uintptr_t)y & 15)) {
+  if (M <= 1 || ((uintptr_t)y & 15) || rows_one_by_one(true, M, K, N)) {
     for (uint32_t m = 0; m < M; m++)
       if (lmhead_q6_k(c, who, x + (size_t)m * K, norm_gamma, eps, planes, y + (size_t)m * N, K, N, GreedyTail{}))
         return -1;

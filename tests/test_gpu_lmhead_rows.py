@@ -186,3 +186,25 @@ def test_rows_weights_beyond_f16(kind):
         g = 1 + prng.randn((K,), 836, std=0.1)
         assert rel2(h.run(x, g), h.ref(x, g)) <= BAR, M
     h.close()
+
+
+@pytest.mark.parametrize("kind", ["q4_0", "q6_k"])
+@pytest.mark.parametrize("M,K,N", [(2, 3072, 1024), (3, 4096, 2048), (5, 8192, 256), (2, 1024, 32768), (16, 3072, 8192)])
+def test_few_rows_time(kind, M, K, N):
+    """A few rows cost no more than through the single-row head (30 % above
+    it: room for the clocks), and agree with it."""
+    h = Head(kind, K, N, 837)
+    x = prng.randn((M, K), 838)
+    us, out = [], []
+    for rows in (True, False):
+        h.run(x, None, rows)
+        device.profile_kernels(True)
+        out.append(h.run(x, None, rows).astype(np.float64))
+        ms, _ = device.profile_read("smith_lmhead_")
+        device.profile_read("")
+        device.profile_kernels(False)
+        us.append(ms * 1e3)
+    print(kind, M, K, N, us)
+    assert us[0] <= 1.3 * us[1], us
+    assert rel2(out[0], out[1]) <= BAR
+    h.close()
