@@ -1424,7 +1424,9 @@ int smith_quantize_q4(void* ctx, const float* w, void* out, uint32_t K, uint32_t
   if (!groups || !N) return 0;
   uint32_t pK = K, pN = N;
   void* args[] = {&w, &out, &pK, &pN};
-  return launch(c, "smith_quantize_q4s", dim3(N / 256 + (N % 256 != 0), std::min<uint32_t>(groups, 65535)), dim3(256),
+  // the groups of a workgroup, as the kernel counts them
+  const uint32_t per = N <= 128 ? 256 / N : 1, rows = groups / per + (groups % per != 0);
+  return launch(c, "smith_quantize_q4s", dim3(N / 256 + (N % 256 != 0), std::min<uint32_t>(rows, 65535)), dim3(256),
                 args);
 }
 

@@ -136,12 +136,15 @@ __device__ __forceinline__ uint32_t q4_exact(float v, double scale, double zero)
 }
 
 // Workgroup (bx, g): 256 columns of group g (grid-stride over the groups), one
-// record a thread.  A thread reads its 32 weights once and holds them; the
-// records leave through LDS as contiguous 8-byte stores.  A quotient is formed
-// in f32 as (v - min) * (15 / range), which is within 6e-6 of the f64 value
-// wherever the latter lies in [0, 15.5] (three f32 roundings of a value <=
-// 15.5, and at most 2^28 * 2^-51 of rounding in the f64 sum, zero being at
-// most 15 * 2^24); only where it comes closer than 1e-4 to a rounding boundary
+// record a thread; of a matrix of 128 columns or fewer, as many whole groups
+// as 256 threads hold (K = 131072, N = 8: 16.4 us with one group each, which
+// left most lanes without a record, 4.9 so).  A thread reads its 32 weights
+// once and holds them; the records leave through LDS as contiguous 8-byte
+// stores.  A quotient is formed in f32 as (v - min) * (15 / range), which is
+// within 6e-6 of the f64 value wherever the latter lies in [0, 15.5] (three
+// f32 roundings of a value <= 15.5, and at most 2^28 * 2^-51 of rounding in
+// the f64 sum, zero being at most 15 * 2^24); only where it comes closer than
+// 1e-4 to a rounding boundary
 // is the f64 division made.  Ranges outside [1e-30, 1e30] (0, infinite,
 // NaN) take the f64 arithmetic throughout.  Memory-bound: K = 4096, N = 14336
 // (279 MB) 50.5 us, 5.5 TB/s; with 33 f64 divisions a record, two reads of the
@@ -153,10 +156,13 @@ extern "C" __global__ __launch_bounds__(QT_COLS) void smith_quantize_q4s(const f
   __shared__ uint2 recs[QT_COLS * 3];
   const uint32_t groups = (K + 31) / 32;
   const uint32_t tid = threadIdx.x, c0 = blockIdx.x * QT_COLS;
+  const uint32_t per = N <= QT_COLS / 2 ? QT_COLS / N : 1;  // groups of a workgroup
   const uint32_t cols = N - c0 < QT_COLS ? N - c0 : QT_COLS;
-  const uint32_t col = c0 + (tid < cols ? tid : cols - 1);
-  for (uint32_t g = blockIdx.y; g < groups; g += gridDim.y) {
-    const uint32_t k0 = g * 32, valid = K - k0 < 32 ? K - k0 : 32;
+  for (uint32_t g0 = blockIdx.y * per; g0 < groups; g0 += gridDim.y * per) {
+    const uint32_t cnt = (groups - g0 < per ? groups - g0 : per) * cols;  // records
+    const uint32_t t = tid < cnt ? tid : cnt - 1, gl = per > 1 ? t / N : 0;
+    const uint32_t col = c0 + t - gl * N;
+    const uint32_t k0 = (g0 + gl) * 32, valid = K - k0 < 32 ? K - k0 : 32;
     const float* src = w + (size_t)k0 * N + col;
     float v[32];
     float mn = __builtin_inff(), mx = -__builtin_inff();  // the values are f32: no rounding in f32 either
@@ -187,23 +193,23 @@ extern "C" __global__ __launch_bounds__(QT_COLS) void smith_quantize_q4s(const f
     const float inv = __fdiv_rn(15.0f, (float)range);
 #pragma unroll
     for (int k = 0; k < 32; k++) {
-      const float t = __fmul_rn(__fsub_rn(v[k], mn), inv);
-      const float c = __builtin_fminf(__builtin_fmaxf(t, 0.f), 15.f);
+      const float u = __fmul_rn(__fsub_rn(v[k], mn), inv);
+      const float c = __builtin_fminf(__builtin_fmaxf(u, 0.f), 15.f);
       const float r = __builtin_rintf(c);
       // |c - r| is the distance to the nearest integer: 0.5 on a boundary;
-      // a NaN t fails the comparison of t with itself
+      // a NaN u fails the comparison of u with itself
       uint32_t q = (uint32_t)r;
-      if (!fast || t != t || !(__builtin_fabsf(c - r) < 0.4999f)) q = q4_exact(v[k], scale, zero);
+      if (!fast || u != u || !(__builtin_fabsf(c - r) < 0.4999f)) q = q4_exact(v[k], scale, zero);
       words[k >> 3] |= q << (4 * (k & 7));
     }
 #pragma unroll
     for (int d = 0; d < 3; d++) recs[tid * 3 + d] = make_uint2(words[2 * d], words[2 * d + 1]);
     __syncthreads();
-    uint2* dst = (uint2*)(out + ((size_t)g * N + c0) * 24);
+    uint2* dst = (uint2*)(out + ((size_t)g0 * N + c0) * 24);
 #pragma unroll
     for (int d = 0; d < 3; d++) {
       const uint32_t i = tid + QT_COLS * d;
-      if (i < cols * 3) dst[i] = recs[i];
+      if (i < cnt * 3) dst[i] = recs[i];
     }
     __syncthreads();
   }

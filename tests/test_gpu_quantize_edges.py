@@ -25,6 +25,38 @@ def test_block_and_group_edges(K, N):
     check(prng.randn((K, N), 811, std=0.02))
 
 
+@pytest.mark.parametrize("K", [32, 63, 8192, 8225])
+@pytest.mark.parametrize("N", [1, 2, 7, 85, 86, 127, 128, 129])
+def test_narrow(K, N):
+    """Several groups to a workgroup up to 128 columns: its last workgroup
+    short of groups, its last group short of rows."""
+    check(prng.randn((K, N), 812, std=0.02))
+
+
+@pytest.mark.parametrize("N", [2, 8])
+def test_narrow_time(N):
+    """A narrow matrix fills the workgroups: quantizing K = 131072 of N columns
+    takes no longer than the same weights as 32 times the columns (1.6 times:
+    its reads are short)."""
+    K = 131072
+    us = []
+    L, ctx = device.lib, device.ops_ctx()
+    w, out = device.alloc(K * N * 4), device.alloc(K // 32 * N * 24)
+    device.check(L.smith_fill_zero(ctx, w, K * N * 4))
+    for k, n in ((K, N), (K // 32, N * 32)):
+        device.check(L.smith_quantize_q4(ctx, w, out, k, n))
+        device.profile_kernels(True)
+        for _ in range(5):
+            device.check(L.smith_quantize_q4(ctx, w, out, k, n))
+        ms, cnt = device.profile_read("smith_quantize_q4s")
+        device.profile_kernels(False)
+        us.append(ms / cnt * 1e3)
+    print(N, us)
+    assert us[0] <= 1.6 * us[1], us
+    for b in (w, out):
+        device.release_buffer(b)
+
+
 @pytest.mark.parametrize("K", [32, 45])
 def test_ties_and_ranges(K):
     rng = np.random.default_rng(812)
