@@ -571,9 +571,11 @@ constexpr size_t NOALLOC_PREP_BYTES = 4u << 20;
 // 2048, 4096 x 14336 both 252.)  Partials take at most 64 MiB, which the
 // context keeps: what 256 workgroups of 256 x 256 tiles take; under 1 % of the
 // shapes up to M = 2048, N = K = 14336 would split further, for 4 % on average.
-// More than 16 splits where one tile or two would leave the chip idle (whole
-// calls, 64 rows: Q6_K 256 x 8192 16 splits 20.1 us, 32 17.8; Q8 64 x 14336 16
-// splits 20.2, 56 17.8).
+// More than 16 splits where few tiles would leave the chip idle (whole calls,
+// 64 rows: Q6_K 256 x 8192 16 splits 20.1 us, 32 17.8; Q8 64 x 14336 16 splits
+// 20.2, 56 17.6), if the estimate gains 15 % and the partials stay within 6
+// MiB: it flatters many short splits (64 rows of Q4_1 1024 x 8192: estimated
+// 16.0 and 13.6, measured 17.4 and 18.5; Q4_0 1024 x 14336 22.1 and 23.6).
 constexpr size_t GEMM3_WS_BYTES = 64u << 20;
 
 uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, bool fused, uint32_t* ks_out) {
@@ -587,6 +589,7 @@ uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, bool fused, uin
     if (tm > 2 && 16 * (tm - 2) >= M) break;  // the tile before holds every row
     const uint64_t tiles = (uint64_t)((M + 16 * tm - 1) / (16 * tm)) * ((N + 255) / 256);
     for (uint32_t ks = 1; (ks <= 16 || (ks <= 64 && tiles * ks <= 256)) && (ks == 1 || S / ks >= 4); ks++) {
+      if (ks > 16 && (size_t)ks * M * N * sizeof(float) > 6u << 20) break;
       const uint32_t sps = (S + ks - 1) / ks;
       if ((S + sps - 1) / sps != ks) continue;  // the same stages per split as a smaller count
       if (ks > 1 && (size_t)ks * M * N * sizeof(float) > GEMM3_WS_BYTES) break;
@@ -597,6 +600,7 @@ uint32_t gemm3_plan(Fmt fmt, uint32_t M, uint32_t N, uint32_t S, bool fused, uin
         break;
       double t = (double)((tiles * ks + 255) / 256) * (sps * (conv + 0.076 * tm) + 3.0 + 0.35 * tm);
       if (ks > 1) t += (fused ? 0.5 : 5.0) + (ks + 1.0) * M * N * 4.0 / 7.2e6;
+      if (ks > 16) t *= 1.17;
       if (t < best) best = t, btm = tm, *ks_out = ks;
     }
   }
