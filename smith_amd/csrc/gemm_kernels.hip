@@ -6,9 +6,13 @@
 //   smith_gemm_prep_a   A (f32, optional RMSNorm with gamma) -> A16 (f16)
 //   smith_gemm_<fmt>_m<BM>_n<BN>  the GEMM, fmt in {q4s, q8, q40, q40t, q41t,
 //                       q50t, q4kt, q6kt}
-//   smith_gemm_prep_a_perm + smith_gemm2_<fmt>_m<BM>_n<BN>  the DMA-staged
-//                       GEMM for the tile-plane formats (further below)
 //   smith_gemm3_<fmt>_m<TM>  the DMA-staged GEMM of every format, K % 64 == 0
+//                       (A as smith_gemm_prep_a_perm leaves it, of Q8 as
+//                       smith_gemm_prep_a does)
+//   smith_gemm2_{q4kt,q6kt}_m128_n64  DMA-staged with narrow tiles, for 65 ..
+//                       128 rows of small Q4_K / Q6_K matrices
+// The register-staged kernels take what is left: K % 64 == 32 (every format
+// but Q4_K / Q6_K) and weights that do not start on a dword.
 //
 // Workgroup tile BM x BN (128x64 .. 256x256), K in stages of BK=64 (two
 // 32-row quantization groups), double-buffered in LDS: while the MFMAs
@@ -386,24 +390,19 @@ DEF_GEMM_FMT(q50t, GT_Q50)
 DEF_GEMM_FMT(q4kt, GT_Q4K)
 DEF_GEMM_FMT(q6kt, GT_Q6K)
 
-// C = epilogue(sum over the ks K-split partials ws[0..ks) [M][N]), fixed
-// order; one thread per output (pair for SwiGLU).
 // ---------------------------------------------------------------------------
-// gemm2: the same GEMM with the operands staged by direct-to-LDS loads
+// gemm2: the same GEMM of Q4_K / Q6_K tiles, 128 rows x 64 columns a
+// workgroup, with the operands staged by direct-to-LDS loads
 // (global_load_lds, no registers on the way) into a ring of 3 stages, and
 // the weights kept in LDS as their raw records -- dequantized in registers
-// right before the MFMAs.  Per stage of 64 K: A rows (f16, 16-byte chunks
-// XOR-swizzled by row through the choice of each lane's source), weight
-// planes of the tile's BN columns for 2 groups (Q4_0 tiles: 16 B of
-// nibbles + 2 B d per record; the other tile formats add their high-bit and
-// parameter planes).  The A operand's 8-element chunks are in the slot order
-// {0,4,1,5,2,6,3,7} (smith_gemm_prep_a_perm), the order in which a nibble
-// dword converts to f16 with 4 bit-inserts (exponent bias 1024 + q for low
-// nibbles, 64 + q for high): both operands permuted alike leave the dot
-// product unchanged.  Q4_0: w = (h - bias - 8) * d in packed f16 (q - 8
-// exact, one rounding).  The loop is unrolled by the ring size so every LDS
-// access names its stage buffer at compile time.  (Q4S records take the
-// register-staged kernel above: converted per wave here they were slower.)
+// right before the MFMAs (gt_weight).  Per stage of 64 K: A rows (f16, 16-byte
+// chunks XOR-swizzled by row through the choice of each lane's source), weight
+// planes of the tile's BN columns for 2 groups.  The A operand's 8-element
+// chunks are in the slot order {0,4,1,5,2,6,3,7} (smith_gemm_prep_a_perm), the
+// order in which a nibble dword converts to f16 with 4 bit-inserts (exponent
+// bias 1024 + q for low nibbles, 64 + q for high): both operands permuted alike
+// leave the dot product unchanged.  The loop is unrolled by the ring size so
+// every LDS access names its stage buffer at compile time.
 // ---------------------------------------------------------------------------
 template <int BYTES_PER_WAVE>
 struct DmaUnit {  // dwordx4 or dword loads splitting a wave's bytes evenly (LDS slot = lane * size)
@@ -433,6 +432,58 @@ struct GtFmt {
   static constexpr int PRM = TILES ? (int)gt_prm_bytes(F) : 0;
   static constexpr int SUP = TILES ? (int)gt_sup_bytes(F) : 0;
 };
+
+// Tile-plane weights 8 kq .. 8 kq + 7 of a record (gguf_tiles.h), in f16 in
+// the slot order {0,4,1,5,2,6,3,7}: w = s*q + c with q exact
+template <int F>
+__device__ __forceinline__ half8 gt_weight(uint32_t x, uint32_t W, uint32_t prm, uint32_t sup, uint32_t kq,
+                                           uint32_t e1024, uint32_t e64) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  const uint32_t y = x >> 8;
+  uint32_t b0 = (x & 0x000F000Fu) | e1024, b1 = (x & 0x00F000F0u) | e64;
+  uint32_t b2 = (y & 0x000F000Fu) | e1024, b3 = (y & 0x00F000F0u) | e64;
+  if constexpr (F == GT_Q50) {
+    // element 8kq + k: bit 4kq + (k & 3) + 16 (k >> 2)
+    b0 |= ((W >> (4 * kq)) << 4) & 0x00100010u;
+    b1 |= ((W >> (4 * kq + 1)) << 8) & 0x01000100u;
+    b2 |= ((W >> (4 * kq + 2)) << 4) & 0x00100010u;
+    b3 |= ((W >> (4 * kq + 3)) << 8) & 0x01000100u;
+  } else if constexpr (F == GT_Q6K) {
+    const uint32_t cb = 4 * (kq & 1);
+    b0 |= ((W >> (2 * cb)) << 4) & 0x00300030u;
+    b1 |= ((W >> (2 * cb + 2)) << 8) & 0x03000300u;
+    b2 |= ((W >> (2 * cb + 4)) << 4) & 0x00300030u;
+    b3 |= ((W >> (2 * cb + 6)) << 8) & 0x03000300u;
+  }
+  h2 sv, cv;
+  if constexpr (F == GT_Q40 || F == GT_Q50) {
+    const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)prm);
+    const _Float16 c = d * (_Float16)(F == GT_Q40 ? -8.0f : -16.0f);  // exact
+    sv = (h2){d, d};
+    cv = (h2){c, c};
+  } else if constexpr (F == GT_Q41) {
+    const h2 dm = __builtin_bit_cast(h2, prm);  // (d, m)
+    sv = (h2){dm.x, dm.x};
+    cv = (h2){dm.y, dm.y};
+  } else {  // Q4_K, Q6_K: f32 products of the f16 and the 6-bit / int8 scales, rounded to f16
+    float s0f, c0f, s1f, c1f;
+    GtW<F> w;
+    w.p = prm;
+    w.sp = sup;
+    gt_affine<F>(w, s0f, c0f, s1f, c1f);
+    const float sf = kq < 2 ? s0f : s1f, cf = kq < 2 ? c0f : c1f;
+    sv = (h2){(_Float16)sf, (_Float16)sf};
+    cv = (h2){(_Float16)cf, (_Float16)cf};
+  }
+  const h2 blo = (h2){(_Float16)1024.0f, (_Float16)1024.0f}, bhi = (h2){(_Float16)64.0f, (_Float16)64.0f};
+  const h2 v0 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b0) - blo, sv, cv);
+  const h2 v1 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b1) - bhi, sv, cv);
+  const h2 v2 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b2) - blo, sv, cv);
+  const h2 v3 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b3) - bhi, sv, cv);
+  const u32x4 u = {__builtin_bit_cast(uint32_t, v0), __builtin_bit_cast(uint32_t, v1),
+                   __builtin_bit_cast(uint32_t, v2), __builtin_bit_cast(uint32_t, v3)};
+  return __builtin_bit_cast(half8, u);
+}
 
 __device__ __forceinline__ constexpr int pad256(int x) { return (x + 255) / 256 * 256; }
 
@@ -479,7 +530,7 @@ __device__ __forceinline__ void gemm2_body(const _Float16* __restrict__ A16, con
                                           float* __restrict__ ws, uint32_t sps) {
   using P = G2<FMT, BM, BN, WM, WN>;
   using GF = GtFmt<FMT>;
-  static_assert(GF::TILES, "tile-plane formats only");
+  static_assert(GF::F == GT_Q4K || GF::F == GT_Q6K, "Q4_K and Q6_K tiles only");
   constexpr int NW = P::NW, WAVES_N = BN / WN;
   constexpr int TM = WM / 16, TN = WN / 16;
   __shared__ __attribute__((aligned(1024))) uint8_t As0[P::A_BYTES], As1[P::A_BYTES], As2[P::A_BYTES];
@@ -498,11 +549,10 @@ __device__ __forceinline__ void gemm2_body(const _Float16* __restrict__ A16, con
   const uint32_t s0 = blockIdx.y * sps < Sall ? blockIdx.y * sps : Sall;
   const uint32_t s1 = s0 + sps < Sall ? s0 + sps : Sall;
   const uint32_t S = s1 - s0;
-  // plane bases (tile formats): Q4_0 tiles take the d plane from D; the
-  // others find their planes after the nibbles (gguf_tiles.h)
+  // plane bases (gguf_tiles.h)
   const GtPlanes PL = gt_planes(GF::F, N, G);
   const uint8_t* hbp = B + PL.hb;
-  const uint8_t* prp = FMT == WF_Q40T ? (const uint8_t*)D : B + PL.prm;
+  const uint8_t* prp = B + PL.prm;
   const uint8_t* sup = B + PL.sup;
   const uint32_t NT16 = N / 16;
   // this wave's DMA instructions per stage
@@ -590,60 +640,15 @@ __device__ __forceinline__ void gemm2_body(const _Float16* __restrict__ A16, con
 #pragma unroll
       for (int j = 0; j < TN; j++) {
         const uint32_t col = wn * WN + j * 16 + r16;
-        u32x4 u;
-        {
-          const uint32_t tt = col / 16, cc = col % 16;
-          const uint32_t ri = (tt * 2 + kk) * 16 + cc;  // record within the stage, tile order
-          const uint32_t x = *(const uint32_t*)(bs + ri * 16 + 4 * kq);
-          const uint32_t y = x >> 8;
-          uint32_t bx = 0x64006400u, by = 0x54005400u, bz = 0x64006400u, bw = 0x54005400u;
-          if constexpr (GF::F == GT_Q50) {
-            const uint32_t W = *(const uint32_t*)(bs + P::NIB + ri * 4);
-            // element 8kq + k: bit 4kq + (k & 3) + 16 (k >> 2) (gguf_tiles.h)
-            bx |= ((W >> (4 * kq)) << 4) & 0x00100010u;
-            by |= ((W >> (4 * kq + 1)) << 8) & 0x01000100u;
-            bz |= ((W >> (4 * kq + 2)) << 4) & 0x00100010u;
-            bw |= ((W >> (4 * kq + 3)) << 8) & 0x01000100u;
-          } else if constexpr (GF::F == GT_Q6K) {
-            const uint2 hw = *(const uint2*)(bs + P::NIB + ri * 8);
-            const uint32_t W = kq < 2 ? hw.x : hw.y, cb = 4 * (kq & 1);
-            bx |= ((W >> (2 * cb)) << 4) & 0x00300030u;
-            by |= ((W >> (2 * cb + 2)) << 8) & 0x03000300u;
-            bz |= ((W >> (2 * cb + 4)) << 4) & 0x00300030u;
-            bw |= ((W >> (2 * cb + 6)) << 8) & 0x03000300u;
-          }
-          // w = s*q + c with q = h - bias exact in f16
-          h2 sv, cv;
-          const uint8_t* prm = bs + P::NIB + P::HBY;
-          if constexpr (GF::F == GT_Q40 || GF::F == GT_Q50) {
-            const _Float16 d = *(const _Float16*)(prm + ri * 2);
-            const _Float16 c = d * (_Float16)(GF::F == GT_Q40 ? -8.0f : -16.0f);  // exact
-            sv = (h2){d, d};
-            cv = (h2){c, c};
-          } else if constexpr (GF::F == GT_Q41) {
-            const h2 dm = *(const h2*)(prm + ri * 4);  // (d, m)
-            sv = (h2){dm.x, dm.x};
-            cv = (h2){dm.y, dm.y};
-          } else {  // Q4_K, Q6_K: f32 products of the f16 and the 6-bit / int8 scales, rounded to f16
-            float s0f, c0f, s1f, c1f;
-            GtW<GF::F> w;
-            w.p = *(const uint16_t*)(prm + ri * 2);
-            w.sp = GF::SUP == 4 ? *(const uint32_t*)(prm + P::PRY + (tt * 16 + cc) * 4)
-                                : *(const uint16_t*)(prm + P::PRY + (tt * 16 + cc) * 2);
-            gt_affine<GF::F>(w, s0f, c0f, s1f, c1f);
-            const float sf = kq < 2 ? s0f : s1f, cf = kq < 2 ? c0f : c1f;
-            sv = (h2){(_Float16)sf, (_Float16)sf};
-            cv = (h2){(_Float16)cf, (_Float16)cf};
-          }
-          const h2 blo = (h2){(_Float16)1024.0f, (_Float16)1024.0f}, bhi = (h2){(_Float16)64.0f, (_Float16)64.0f};
-          const h2 v0 = __builtin_elementwise_fma(__builtin_bit_cast(h2, (x & 0x000F000Fu) | bx) - blo, sv, cv);
-          const h2 v1 = __builtin_elementwise_fma(__builtin_bit_cast(h2, (x & 0x00F000F0u) | by) - bhi, sv, cv);
-          const h2 v2 = __builtin_elementwise_fma(__builtin_bit_cast(h2, (y & 0x000F000Fu) | bz) - blo, sv, cv);
-          const h2 v3 = __builtin_elementwise_fma(__builtin_bit_cast(h2, (y & 0x00F000F0u) | bw) - bhi, sv, cv);
-          u = (u32x4){__builtin_bit_cast(uint32_t, v0), __builtin_bit_cast(uint32_t, v1),
-                      __builtin_bit_cast(uint32_t, v2), __builtin_bit_cast(uint32_t, v3)};
-        }
-        bf[j] = __builtin_bit_cast(half8, u);
+        const uint32_t tt = col / 16, cc = col % 16;
+        const uint32_t ri = (tt * 2 + kk) * 16 + cc;  // record within the stage, tile order
+        const uint32_t x = *(const uint32_t*)(bs + ri * 16 + 4 * kq);
+        const uint32_t hw = GF::HB ? *(const uint32_t*)(bs + P::NIB + ri * 8 + 4 * (kq >> 1)) : 0u;
+        const uint8_t* prm = bs + P::NIB + P::HBY;
+        const uint32_t pw = *(const uint16_t*)(prm + ri * 2);
+        const uint32_t sw = GF::SUP == 4 ? *(const uint32_t*)(prm + P::PRY + (tt * 16 + cc) * 4)
+                                         : *(const uint16_t*)(prm + P::PRY + (tt * 16 + cc) * 2);
+        bf[j] = gt_weight<GF::F>(x, hw, pw, sw, kq, 0x64006400u, 0x54005400u);
       }
 #pragma unroll
       for (int i = 0; i < TM; i++)
@@ -698,19 +703,11 @@ __device__ __forceinline__ void gemm2_body(const _Float16* __restrict__ A16, con
       float* __restrict__ ws, uint32_t sps) {                                                                \
     gemm2_body<FMT, BM, BN, WM, WN>(A16, B, D, C, M, N, K, R, epi, ws, sps);                                  \
   }
-// 128-row tiles: four waves side by side along N, each over all 128 rows,
-// so every B fragment is converted once per workgroup (two 64-row waves per
-// column converted it twice: gate|up at M = 128 36.7 -> 34.6 us)
-#define DEF_GEMM2_FMT(TAG, FMT)                                   \
-  DEF_GEMM2(smith_gemm2_##TAG##_m128_n64, FMT, 128, 64, 128, 16)   \
-  DEF_GEMM2(smith_gemm2_##TAG##_m128_n128, FMT, 128, 128, 128, 32) \
-  DEF_GEMM2(smith_gemm2_##TAG##_m256_n128, FMT, 256, 128, 64, 64) \
-  DEF_GEMM2(smith_gemm2_##TAG##_m256_n256, FMT, 256, 256, 64, 64)
-DEF_GEMM2_FMT(q40t, WF_Q40T)
-DEF_GEMM2_FMT(q41t, GT_Q41)
-DEF_GEMM2_FMT(q50t, GT_Q50)
-DEF_GEMM2_FMT(q4kt, GT_Q4K)
-DEF_GEMM2_FMT(q6kt, GT_Q6K)
+// Four waves side by side along N, each over all 128 rows, so every B
+// fragment is converted once per workgroup (two 64-row waves per column
+// converted it twice: gate|up at M = 128 36.7 -> 34.6 us)
+DEF_GEMM2(smith_gemm2_q4kt_m128_n64, GT_Q4K, 128, 64, 128, 16)
+DEF_GEMM2(smith_gemm2_q6kt_m128_n64, GT_Q6K, 128, 64, 128, 16)
 
 // ---------------------------------------------------------------------------
 // gemm3: the GEMM on (g, n) records (Q4S, Q8, Q4_0 planes) and on the GGUF
@@ -745,9 +742,12 @@ DEF_GEMM2_FMT(q6kt, GT_Q6K)
 // write: it would wait for every load in flight before the next LDS read.
 // There is no destination register, and the kernel counts the loads itself
 // (s_waitcnt vmcnt before the barrier that publishes a stage).  One wait
-// state between the write of M0 and its use.  The compiler warns that M0 is
-// reserved: it must not keep a value there across this, and the emitted code
-// of the kernels that call it uses M0 nowhere else.
+// state between the write of M0 and its use.  The compiler warns, once per
+// load, that M0 is reserved (silenced here alone): it must not keep a value
+// there across this, and the emitted code of the kernels that call it uses M0
+// nowhere else.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint32_t lds) {
   asm volatile(
       "s_mov_b32 m0, %0\n\t"
@@ -757,6 +757,7 @@ __device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint32_
       : "s"(lds), "v"(off), "s"(base)
       : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 // a wave-uniform 64-bit value in scalar registers
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
@@ -813,58 +814,6 @@ struct G3Raw {
   float s, z;
   uint32_t h, p, sp;  // tile planes: high bits (the word of this K slice), prm, sup
 };
-
-// Tile-plane weights 8 kq .. 8 kq + 7 of a record (gguf_tiles.h), in f16 in
-// the slot order {0,4,1,5,2,6,3,7}: w = s*q + c with q exact
-template <int F>
-__device__ __forceinline__ half8 gt_weight(uint32_t x, uint32_t W, uint32_t prm, uint32_t sup, uint32_t kq,
-                                           uint32_t e1024, uint32_t e64) {
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  const uint32_t y = x >> 8;
-  uint32_t b0 = (x & 0x000F000Fu) | e1024, b1 = (x & 0x00F000F0u) | e64;
-  uint32_t b2 = (y & 0x000F000Fu) | e1024, b3 = (y & 0x00F000F0u) | e64;
-  if constexpr (F == GT_Q50) {
-    // element 8kq + k: bit 4kq + (k & 3) + 16 (k >> 2)
-    b0 |= ((W >> (4 * kq)) << 4) & 0x00100010u;
-    b1 |= ((W >> (4 * kq + 1)) << 8) & 0x01000100u;
-    b2 |= ((W >> (4 * kq + 2)) << 4) & 0x00100010u;
-    b3 |= ((W >> (4 * kq + 3)) << 8) & 0x01000100u;
-  } else if constexpr (F == GT_Q6K) {
-    const uint32_t cb = 4 * (kq & 1);
-    b0 |= ((W >> (2 * cb)) << 4) & 0x00300030u;
-    b1 |= ((W >> (2 * cb + 2)) << 8) & 0x03000300u;
-    b2 |= ((W >> (2 * cb + 4)) << 4) & 0x00300030u;
-    b3 |= ((W >> (2 * cb + 6)) << 8) & 0x03000300u;
-  }
-  h2 sv, cv;
-  if constexpr (F == GT_Q40 || F == GT_Q50) {
-    const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)prm);
-    const _Float16 c = d * (_Float16)(F == GT_Q40 ? -8.0f : -16.0f);  // exact
-    sv = (h2){d, d};
-    cv = (h2){c, c};
-  } else if constexpr (F == GT_Q41) {
-    const h2 dm = __builtin_bit_cast(h2, prm);  // (d, m)
-    sv = (h2){dm.x, dm.x};
-    cv = (h2){dm.y, dm.y};
-  } else {  // Q4_K, Q6_K: f32 products of the f16 and the 6-bit / int8 scales, rounded to f16
-    float s0f, c0f, s1f, c1f;
-    GtW<F> w;
-    w.p = prm;
-    w.sp = sup;
-    gt_affine<F>(w, s0f, c0f, s1f, c1f);
-    const float sf = kq < 2 ? s0f : s1f, cf = kq < 2 ? c0f : c1f;
-    sv = (h2){(_Float16)sf, (_Float16)sf};
-    cv = (h2){(_Float16)cf, (_Float16)cf};
-  }
-  const h2 blo = (h2){(_Float16)1024.0f, (_Float16)1024.0f}, bhi = (h2){(_Float16)64.0f, (_Float16)64.0f};
-  const h2 v0 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b0) - blo, sv, cv);
-  const h2 v1 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b1) - bhi, sv, cv);
-  const h2 v2 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b2) - blo, sv, cv);
-  const h2 v3 = __builtin_elementwise_fma(__builtin_bit_cast(h2, b3) - bhi, sv, cv);
-  const u32x4 u = {__builtin_bit_cast(uint32_t, v0), __builtin_bit_cast(uint32_t, v1),
-                   __builtin_bit_cast(uint32_t, v2), __builtin_bit_cast(uint32_t, v3)};
-  return __builtin_bit_cast(half8, u);
-}
 
 template <int FMT, int TM>
 __device__ __forceinline__ void gemm3_body(const _Float16* __restrict__ A16, const uint8_t* __restrict__ B,
@@ -1187,7 +1136,7 @@ __device__ __forceinline__ void prep_a_row(const float* __restrict__ A, const fl
                                            _Float16* __restrict__ A16, uint32_t K);
 
 // A16 as smith_gemm_prep_a, with each 8-element chunk in the slot order
-// {0,4,1,5,2,6,3,7} of the gemm2 weight conversion.
+// {0,4,1,5,2,6,3,7} of the nibble conversions (q4_pairs, gt_weight).
 extern "C" __global__ __launch_bounds__(256) void smith_gemm_prep_a_perm(const float* __restrict__ A,
                                                                         const float* __restrict__ gamma, float eps,
                                                                         _Float16* __restrict__ A16, uint32_t K) {

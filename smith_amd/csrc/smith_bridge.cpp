@@ -618,25 +618,18 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
                    c->a16_bytes >= (size_t)M * K * 2;
   c->a16_src = nullptr;
   if (ensure(c, &c->a16, &c->a16_bytes, (size_t)M * K * 2)) return -1;
-  // tile-plane formats (Q4_0 tiles, Q4_1, Q5_0, Q4_K, Q6_K) with K % 64 == 0:
-  // the DMA-staged kernels (smith_gemm2_*),
-  // whose A operand is in the permuted slot order.  (On Q4S records the f32
-  // in-register dequantisation, repeated by the waves sharing a weight
-  // fragment, made them slower at config-4 sizes: 487 vs 331 us.)
-  static const bool gemm2_on = [] {
-    const char* e = getenv("SMITH_GEMM2");
-    return !(e && e[0] == '0');
-  }();
-  const bool g2 = gemm2_on && (fmt == FQ40T || fmt >= FQ41T) && K % 64 == 0;
-  // K % 64 == 0: smith_gemm3_* (dword-aligned records and planes; the scales
-  // of Q4_0 records may start at any f16).  Q4_K / Q6_K tiles of 65 .. 128
-  // rows and fewer than 8192 columns keep smith_gemm2_*, whose 64-column
-  // tiles need fewer K splits there (whole calls, 128 rows, gemm2 / gemm3:
-  // Q6_K 3072 x 9216 31.9 / 32.9 us, Q4_K 3072 x 3072 22.2 / 22.4; against
-  // Q4_K 18432 x 3072 41.4 / 36.7, and 3072 x 3072 at 64 rows 17.7 / 16.4).
-  const bool k128 = g2 && (fmt == FQ4KT || fmt == FQ6KT) && M > 64 && M <= 128 && N < 8192;
-  const bool g3 = K % 64 == 0 && !k128 && ((uintptr_t)B & (fmt == FQ8 ? 1 : 3)) == 0 &&
-                  ((uintptr_t)D & (fmt == FQ40 ? 1 : 3)) == 0;
+  // K % 64 == 0: smith_gemm3_*, on dword-aligned records and planes (the
+  // scales of Q4_0 records may start at any f16).  Q4_K / Q6_K tiles of 65 ..
+  // 128 rows of a small matrix take smith_gemm2_*, whose 64-column tiles need
+  // fewer K splits there (whole calls, gemm2 / gemm3 at 65 and at 128 rows:
+  // Q4_K 3072 x 3072 18.1 / 19.0, 22.2 / 23.3 us; 4096 x 4096 22.8 / 24.8, 25.8
+  // / 25.7; 4096 x 6144 26.9 / 25.5, 27.1 / 25.5; 8176 x 8192 43.5 / 33.6, 44.0
+  // / 37.6.  Q6_K 3072 x 3072 19.1 / 21.1, 22.9 / 24.4; 8176 x 3072 25.1 /
+  // 24.3, 27.4 / 28.2; 4096 x 8192 31.6 / 27.2, 33.1 / 32.8).
+  const bool dma = K % 64 == 0 && ((uintptr_t)B & (fmt == FQ8 ? 1 : 3)) == 0 && ((uintptr_t)D & (fmt == FQ40 ? 1 : 3)) == 0;
+  const bool g2 = dma && (fmt == FQ4KT || fmt == FQ6KT) && M > 64 && M <= 128 && N < 8192 &&
+                  (uint64_t)N * K < (fmt == FQ4KT ? 24u << 20 : 32u << 20);
+  const bool g3 = dma && !g2;
   {
     const float* pa = a;
     const float* pg = ep.gamma;
@@ -644,8 +637,7 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
     void* pd = c->a16;
     uint32_t pK = K;
     void* args[] = {&pa, &pg, &pe, &pd, &pK};
-    // the DMA-staged kernels and the register-staged Q4S / Q4_0 ones take A
-    // in the permuted slot order of their packed-f16 weight conversion
+    // the packed-f16 nibble conversions take A in their permuted slot order
     const bool perm = g2 || (g3 && fmt != FQ8) || fmt == FQ4S || fmt == FQ40 || fmt == FQ40T;
     if (!(pre && perm) && launch(c, perm ? "smith_gemm_prep_a_perm" : "smith_gemm_prep_a", dim3(M), dim3(256), args))
       return -1;
@@ -663,20 +655,19 @@ int gemm(Ctx* c, Fmt fmt, const float* a, const void* B, const void* D, float* o
     // (bigger tiles carry more MFMA work per K stage to cover load latency);
     // small grids split K across workgroups (partials reduced after)
     uint32_t bm = 128, bn = 64;
-    if (ntiles(256, 256) >= 256) bm = 256, bn = 256;
-    else if (ntiles(256, 128) >= 200) bm = 256, bn = 128;
-    else if (ntiles(128, 128) >= 256) bm = 128, bn = 128;
-    if (g2 && M <= 128) bn = ntiles(128, 128) >= 128 ? 128 : 64;
-    if (g2 && bm == 256 && bn == 256) bn = 128;  // 256x256 spills registers on the high-bit formats
-    // M >= 256 on the register-staged kernel: 256x256 tiles (one 1024-thread
-    // workgroup per CU) and enough K splits to fill one wave of workgroups,
-    // each split at least 8 stages
-    const bool big = !g2 && M >= 256;
+    if (!g2) {
+      if (ntiles(256, 256) >= 256) bm = 256, bn = 256;
+      else if (ntiles(256, 128) >= 200) bm = 256, bn = 128;
+      else if (ntiles(128, 128) >= 256) bm = 128, bn = 128;
+    }
+    // M >= 256: 256x256 tiles (one 1024-thread workgroup per CU) and enough K
+    // splits to fill one wave of workgroups, each split at least 8 stages
+    const bool big = M >= 256;
     if (big) bm = bn = 256;
     tiles = ntiles(bm, bn);
     if (big) {
       ks = std::max<uint32_t>(1, std::min<uint32_t>(256 / tiles, S / 8));
-    } else if (g2 && bm == 128 && tiles < 512) {
+    } else if (g2) {
       // about 450 workgroups, at least 6 stages per split (measured at M = 128)
       ks = std::min<uint32_t>(std::max<uint32_t>(1, (448 + tiles / 2) / tiles), std::max<uint32_t>(1, S / 6));
     } else if (bm == 128 && bn == 64 && tiles < 512) {

@@ -68,8 +68,9 @@ def test_code_object_has_kernels():
     for k in ["smith_gemm_prep_a", "smith_gemm_prep_a_perm", "smith_gemm_reduce"] + [
             "smith_gemm_%s_m%d_n%d" % (f, m, n) for f in ("q4s", "q8", "q40", "q40t", "q41t", "q50t", "q4kt", "q6kt")
             for (m, n) in ((128, 64), (128, 128), (256, 128), (256, 256))] + [
-            "smith_gemm2_%s_m%d_n%d" % (f, m, n) for f in ("q40t", "q41t", "q50t", "q4kt", "q6kt")
-            for (m, n) in ((128, 64), (128, 128), (256, 128), (256, 256))]:
+            "smith_gemm2_%s_m128_n64" % f for f in ("q4kt", "q6kt")] + [
+            "smith_gemm3_%s_m%d" % (f, m) for f in ("q4s", "q8", "q40", "q40t", "q41t", "q50t", "q4kt", "q6kt")
+            for m in (2, 4, 6, 8, 10, 12, 14, 16) if m > 2 or f.endswith("t")]:
         assert re.search(r"\b%s\.kd\b" % k, out), k
     out = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--syms", device.LLAMA_CODE_OBJECT_PATH],
                          capture_output=True, text=True, check=True).stdout
