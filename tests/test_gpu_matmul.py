@@ -465,12 +465,13 @@ def test_config4_prefill_gemm(N, K):
     assert e <= TOL_GEMM, e
 
 
-# ---------------- M >= 256: 256x256 tiles with K splits ----------------
+# ---------------- M >= 256, K % 64 == 0: K splits ----------------
 
 @pytest.mark.parametrize("M,K,N", [(300, 4096, 300), (257, 1024, 520), (512, 14336, 96), (257, 2048, 18)])
 def test_gemm_big_tiles_ragged(M, K, N):
-    """M >= 256 runs 256x256 tiles with enough K splits to fill the chip
-    (8 / 2 / 8 splits here) over ragged row and column tiles, Q4S and Q8."""
+    """smith_gemm3_* in 64-row tiles with enough K splits to fill the chip over
+    ragged row and column tiles, Q4S and Q8 (K % 64 == 32, the register-staged
+    256x256 tiles: test_register_staged in test_gpu_gemm3.py)."""
     w = prng.randn((K, N), 61, std=0.02)
     a = prng.randn((M, K), 62)
     q = S.quantizeQ4(w)
@@ -484,9 +485,8 @@ def test_gemm_big_tiles_ragged(M, K, N):
 @pytest.mark.parametrize("epi", [1, 2])
 @pytest.mark.parametrize("K", [2048, 1024])
 def test_gemm_big_tiles_epilogues(epi, K):
-    """The K-split finish applies the residual / SwiGLU epilogue (Q8 linear
-    with a fused RMSNorm, M = 300 rows on 256x256 tiles): 4 splits summed by
-    smith_gemm_reduce (K = 2048) and 2 (K = 1024)."""
+    """The K-split finish (smith_gemm_reduce) applies the residual / SwiGLU
+    epilogue: Q8 linear with a fused RMSNorm, M = 300 rows on smith_gemm3_*."""
     M, N, eps = 300, 320, 1e-5
     w = prng.randn((K, N), 63, std=0.02)
     x = prng.randn((M, K), 64)
