@@ -345,8 +345,8 @@ int smith_lmhead_q4_0_greedy(void* ctx, const float* x, const float* norm_gamma,
                              uint32_t wk, float* rope_row);
 /* The LM heads above for M rows of x (row length K) at once: y is [M][N], the
  * logits of a prompt's rows.  f32 accuracy (split f16 operands on the matrix
- * cores, f32 where a result is not finite); one row runs the single-row
- * kernel.  Same shape rules as smith_lmhead_q4_0_nb / smith_lmhead_q6_k_nb. */
+ * cores, f32 where a result is not finite); one row, and a few rows where that
+ * is faster, run the single-row kernel.  Same shape rules as smith_lmhead_q4_0_nb / smith_lmhead_q6_k_nb. */
 int smith_lmhead_q4_0_rows(void* ctx, const float* x, uint32_t M, const float* norm_gamma, float eps, const void* nib,
                            const void* d, float* y, uint32_t K, uint32_t N);
 int smith_lmhead_q6_k_rows(void* ctx, const float* x, uint32_t M, const float* norm_gamma, float eps,

@@ -733,9 +733,9 @@ DEF_GEMM2(smith_gemm2_q6kt_m128_n64, GT_Q6K, 128, 64, 128, 16)
 // Measured (whole call: activation prep, GEMM, K-split reduce; the register-
 // staged kernel before it): Q4S M = 512, 14336 x 4096 80 -> 66 us; M = 2048,
 // 4096 x 14336 259 -> 242 us; Q8 M = 301, 14336 x 4096 84 -> 57 us; against
-// smith_gemm2_*: Q4_K 28672 x 4096 at 2 / 128 / 250 rows 115 -> 29, 119 -> 53,
-// 121 -> 79 us, Q6_K 4096 x 14336 42 -> 25, 49 -> 42, 74 -> 62 us, Q4_0 18432
-// x 3072 at 250 rows 76 -> 45 us.
+// the gemm2 tiles that it replaced: Q4_K 28672 x 4096 at 2 / 128 / 250 rows 115
+// -> 29, 119 -> 53, 121 -> 79 us, Q6_K 4096 x 14336 42 -> 25, 49 -> 42, 74 ->
+// 62 us, Q4_0 18432 x 3072 at 250 rows 76 -> 45 us.
 // ---------------------------------------------------------------------------
 // 16 bytes per lane from base + off (a lane's own) to LDS byte address lds +
 // 16 * lane (wave-uniform).  In asm so that the compiler does not see an LDS

@@ -563,9 +563,10 @@ constexpr size_t NOALLOC_PREP_BYTES = 4u << 20;
 // Row tiles per workgroup (TM) and K splits of smith_gemm3_*: the pair with
 // the least estimated time.  256 workgroups run at once (one a CU); a stage
 // of K = 64 takes about 0.35 + 0.076 TM us (0.45 for the formats with a longer
-// conversion: Q8, Q4_1 and on), filling the ring and storing the tile 3 + 0.35 TM us, and splits add
-// the reduce: partials read and result written at 7.2 TB/s, and 5 us (fused:
-// it also prepares the next GEMM's rows, a launch less there, and 0.5 us).
+// conversion: Q8, Q4_1 and on), filling the ring and storing the tile 3 + 0.35
+// TM us, and splits add the reduce: partials read and result written at 7.2
+// TB/s, and 5 us (fused: it also prepares the next GEMM's rows, a launch less
+// there, and 0.5 us).
 // (Measured on either side: Q4S M = 512, 14336 x 4096 TM = 8 without splits
 // 71 us, 16 with two 81; Q8 M = 301 10 with two 61, 8 without 69; Q4S M =
 // 2048, 4096 x 14336 both 252.)  Partials take at most 64 MiB, which the
@@ -814,11 +815,12 @@ static int noalloc_setup(Ctx* c) {
 
 // Large device -> host copies into ordinary memory: the runtime's own way is
 // one chunk at a time, the device idle while the host copies it out of its
-// staging (16.4 MB into fresh memory 930 us, here 608; 4 MB 242 / 226).  Eight pinned 1 MB slots: the copies
-// into them run ahead on the context's stream and the calling thread with
-// three helpers moves them on.  The helpers sleep until the first slot is
-// full: work that the stream has to do before keeps only the calling thread
-// waiting, as a plain copy does.  Below 4 MB the helpers cost what they save.
+// staging (16.4 MB into fresh memory 930 us, here 608; 4 MB 242 / 226).  Eight
+// pinned 1 MB slots: the copies into them run ahead on the context's stream and
+// the calling thread with three helpers moves them on.  The helpers sleep until
+// the first slot is full: work that the stream has to do before keeps only the
+// calling thread waiting, as a plain copy does.  Below 4 MB the helpers cost
+// what they save.
 constexpr uint64_t STAGE_CHUNK = 1u << 20, STAGE_MIN_BYTES = 4u << 20;
 constexpr int STAGE_SLOTS = 8, STAGE_HELPERS = 3;
 
