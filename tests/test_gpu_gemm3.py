@@ -229,6 +229,27 @@ def test_register_staged_tiles(t, tile, M, N, K):
     w.close()
 
 
+@pytest.mark.parametrize("t", [O.GGML_Q4_0, O.GGML_Q4_1, O.GGML_Q5_0, O.GGML_Q4_K, O.GGML_Q6_K])
+@pytest.mark.parametrize("M", [66, 130])
+def test_planes_off_a_dword(t, M):
+    """Planes that start two bytes past a dword take the register-staged
+    kernel (the DMA needs dwords)."""
+    N, K = 48, 512
+    tag = {O.GGML_Q4_0: "q40t", O.GGML_Q4_1: "q41t", O.GGML_Q5_0: "q50t", O.GGML_Q4_K: "q4kt", O.GGML_Q6_K: "q6kt"}[t]
+    w = Tiles(t, N, K, 733)
+    raw = device.download(w.planes, int(device.lib.smith_gguf_tiles_bytes(t, N, K)), np.uint8)
+    base = device.alloc(raw.size + 64)
+    device.upload(base, np.concatenate([np.zeros(2, np.uint8), raw, np.zeros(62, np.uint8)]))
+    a = prng.randn((M, K), 734)
+    at, out = S.tensor(a), S.create([M, N])
+    with launched("smith_gemm_%s_m128_n64" % tag):
+        device.check(device.lib.smith_linear_gguf_tiles(device.ops_ctx(), t, at.buffer, base + 2, out.buffer, M, N, K,
+                                                        None, 0.0, None, 0))
+    assert rel2(out.data, a.astype(np.float64) @ w.w.T) <= BAR
+    device.release_buffer(base)
+    w.close()
+
+
 @pytest.mark.parametrize("fmt", ["q8", "q40"])
 @pytest.mark.parametrize("epi", [1, 2])
 @pytest.mark.parametrize("M,N,K", [(300, 320, 1056), (300, 322, 480), (130, 66, 1056)])
