@@ -4,7 +4,7 @@
  * TEST INFRASTRUCTURE ONLY.  Nothing in the product (smith_amd/, include/,
  * the HIP kernels) links, loads or calls this file.  Only tests/,
  * __graft_entry__.smoke() and bench.py's cpu_baseline leg use it, and only as
- * the checker / the timed CPU baseline.
+ * the oracle of the tests / the timed CPU baseline.
  *
  * Build: make -C oracle   (plain C11, -O2 -ffp-contract=off, no fast-math)
  *

@@ -25,7 +25,7 @@ LIBSMITH = os.path.join(LIBDIR, "libsmith.so")
 HSACO_BENCH = os.path.join(LIBDIR, "smith_bench.hsaco")
 LIBBENCH = os.path.join(LIBDIR, "libsmith_bench.so")
 
-# -packed-fp32-ops: never emit v_pk_{add,mul,fma}_f32 (unreliable on the pool).
+# -packed-fp32-ops: never emit v_pk_{add,mul,fma}_f32 (some of their forms have given wrong results).
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
